@@ -20,9 +20,11 @@ SAS_META_SIZE = 1024
 SAS_FWD_NO_COMBINE = 1
 SAS_BWD_WINDOW_TOKENS = 2   # backward: per-token adds for window rows
 SAS_BWD_WINDOW_KEYS = 4     # backward: the key-major window pass
+SAS_BWD_WORKSPACE = 8       # backward: fwd.workspace holds sas_bwd_plan's bytes
+SAS_BWD_DQ_DTYPE = 16       # backward: dq in the query dtype, written whole
 
 EXPORTED = ("sas_metadata_v1", "sas_metadata_device_v1", "sas_fwd_plan", "sas_fwd_v1", "sas_fwd_noalloc_v1", "sas_combine_v1",
-            "sas_cache_write_v1", "sas_bwd_v1", "sas_last_error", "sas_version",
+            "sas_cache_write_v1", "sas_bwd_v1", "sas_bwd_plan", "sas_last_error", "sas_version",
             "sas_bench_atomic_add_v1")
 
 _i32p = C.POINTER(C.c_int32)
@@ -122,6 +124,8 @@ def lib() -> C.CDLL:
                 L.sas_combine_v1.restype = C.c_int
                 L.sas_bwd_v1.argtypes = [C.POINTER(SasBwdArgs), C.c_void_p]
                 L.sas_bwd_v1.restype = C.c_int
+                L.sas_bwd_plan.argtypes = [C.POINTER(SasBwdArgs), _i32p, C.POINTER(C.c_size_t)]
+                L.sas_bwd_plan.restype = C.c_int
                 L.sas_cache_write_v1.argtypes = [C.POINTER(SasCacheWriteArgs), C.c_void_p]
                 L.sas_cache_write_v1.restype = C.c_int
                 L.sas_bench_atomic_add_v1.argtypes = [C.c_void_p, C.c_int32, C.c_int32, C.c_int32, C.c_int32,

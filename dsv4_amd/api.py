@@ -759,6 +759,13 @@ def prepare_sparse_attn_sharedkv_backward(dout: torch.Tensor, q: torch.Tensor, o
     add per 16 heads, beside the per-token kernel on a side stream); False,
     one add per (token, row); the results agree up to fp32 summation
     order."""
+    return _prepare_backward(dout, q, out, lse, False, **kwargs)
+
+
+def _prepare_backward(dout, q, out, lse, own_dq: bool, **kwargs) -> PreparedBackward:
+    """``own_dq``: dq may be a fresh tensor in q's dtype, written whole by one
+    launch, where the library's plan writes it so (no fp32 buffer to clear
+    and convert)."""
     kwargs.pop("return_softmax_lse", None)
     window_pass = kwargs.pop("window_pass", None)
     call = prepare_sparse_attn_sharedkv(q, **kwargs)
@@ -783,7 +790,20 @@ def prepare_sparse_attn_sharedkv_backward(dout: torch.Tensor, q: torch.Tensor, o
     dout_f, out_f, lse_f = dout_f.contiguous(), out_f.contiguous(), lse_f.contiguous()
     ori_kv = kwargs["ori_kv"]
     cmp_kv = kwargs.get("cmp_kv")
-    dq = torch.zeros((T1, H, int(a.D)), dtype=torch.float32, device=dev)
+    keep = [dout_f, out_f, lse_f]
+    direct, ws = C.c_int32(0), C.c_size_t(0)
+    _lib.check(_lib.lib().sas_bwd_plan(C.byref(_lib.SasBwdArgs(fwd=a)), C.byref(direct), C.byref(ws)),
+               "sparse_attn_sharedkv_backward")
+    if ws.value:
+        work = torch.empty(ws.value, dtype=torch.uint8, device=dev)
+        keep.append(work)
+        a.flags |= _lib.SAS_BWD_WORKSPACE
+        a.workspace, a.workspace_bytes = work.data_ptr(), ws.value
+    if own_dq and direct.value:
+        a.flags |= _lib.SAS_BWD_DQ_DTYPE
+        dq = torch.empty((T1, H, int(a.D)), dtype=q.dtype, device=dev)
+    else:
+        dq = torch.zeros((T1, H, int(a.D)), dtype=torch.float32, device=dev)
     d_ori = torch.zeros(ori_kv.shape, dtype=torch.float32, device=dev)
     d_cmp = torch.zeros(cmp_kv.shape, dtype=torch.float32, device=dev) if cmp_kv is not None else None
     d_sinks = torch.zeros(H, dtype=torch.float32, device=dev)
@@ -791,7 +811,7 @@ def prepare_sparse_attn_sharedkv_backward(dout: torch.Tensor, q: torch.Tensor, o
     ba = _lib.SasBwdArgs(fwd=a, dout=dout_f.data_ptr(), dq=dq.data_ptr(), d_ori_kv=d_ori.data_ptr(),
                          d_cmp_kv=d_cmp.data_ptr() if d_cmp is not None else None,
                          d_sinks=d_sinks.data_ptr())
-    return PreparedBackward(call, ba, [dout_f, out_f, lse_f], q, dq, d_ori, d_cmp, d_sinks)
+    return PreparedBackward(call, ba, keep, q, dq, d_ori, d_cmp, d_sinks)
 
 
 def sparse_attn_sharedkv_backward(
@@ -813,7 +833,7 @@ def sparse_attn_sharedkv_backward(
     ``[H]``. Key sets are the forward's: window rows and the valid top-k (or
     dense compressed) rows; V is the first 512 channels of each row.
     """
-    pb = prepare_sparse_attn_sharedkv_backward(dout, q, out, lse, **kwargs)
+    pb = _prepare_backward(dout, q, out, lse, True, **kwargs)
     pb.launch()
     return pb.result()
 

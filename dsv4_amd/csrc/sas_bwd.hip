@@ -28,10 +28,8 @@
 // 16x16x16 MFMAs per 16-channel tile.
 
 #include <mutex>
-#include <type_traits>
-#include <utility>
 
-#include "sas_kern.h"
+#include "sas_bwd.h"
 
 namespace sas {
 namespace {
@@ -43,63 +41,6 @@ constexpr int kBwdRows = 16;   // rows per chunk (= lanes per head)
 #ifndef SAS_BWD64
 #define SAS_BWD64 1    // 1: 64-head workgroups (sas_bwd64_kernel) when H is a multiple of 64
 #endif
-
-struct BwdParams {
-  FwdParams f;
-  const uint8_t* out;   // [T, H, 512] q dtype
-  const uint8_t* dout;  // [T, H, 512] q dtype
-  float* dq;            // [T, H, D] fp32
-  float* d_ori;         // [ori rows, D] fp32, accumulated
-  float* d_cmp;         // [cmp rows, D] fp32, accumulated (null for SWA)
-  float* d_sinks;       // [H] fp32, accumulated
-  int win_pass;         // 1: window rows' gradients come from sas_bwd_win_kernel (the per-token kernels skip them)
-  int win_tiles;        // sas_bwd_win_kernel: 64-position row tiles per batch
-};
-
-// f(integral_constant<int, j>) for j = 0 .. N-1, with no loop: arrays
-// indexed this way are split into registers, while an array indexed inside a
-// loop (even one unrolled later) is first moved to LDS or scratch memory by
-// the compiler, which made each row-chunk prefetch a load waited for at once.
-template <typename F, int... I>
-__device__ __forceinline__ void unroll_impl(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void unroll(F&& f) {
-  unroll_impl(f, std::make_integer_sequence<int, N>{});
-}
-template <typename QT>
-__device__ __forceinline__ float to_f(uint16_t v) {
-  return (float)__builtin_bit_cast(QT, v);
-}
-
-// c + a.x * b.x + a.y * b.y for two packed 16-bit pairs (v_dot2c_f32_bf16 /
-// v_dot2c_f32_f16)
-template <typename QT>
-__device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
-  typedef QT v2 __attribute__((ext_vector_type(2)));
-  if constexpr (std::is_same<QT, __bf16>::value)
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2, a), __builtin_bit_cast(v2, b), c, false);
-  else
-    return __builtin_amdgcn_fdot2(__builtin_bit_cast(v2, a), __builtin_bit_cast(v2, b), c, false);
-}
-
-// two packed 16-bit values (low half first) -> floats
-template <typename QT>
-__device__ __forceinline__ float2 unpack2(uint32_t w) {
-  return make_float2(to_f<QT>((uint16_t)(w & 0xffffu)), to_f<QT>((uint16_t)(w >> 16)));
-}
-
-// Sum over the 16 lanes of a DPP row (a head's lanes), returned in every
-// lane: quad_perm [1,0,3,2] and [2,3,0,1] (lane xor 1, xor 2), then
-// row_half_mirror and row_mirror pair the quads and the halves.
-__device__ __forceinline__ float sum16(float x) {
-  x += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0xB1, 0xF, 0xF, false));
-  x += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x4E, 0xF, 0xF, false));
-  x += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x141, 0xF, 0xF, false));
-  x += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x140, 0xF, 0xF, false));
-  return x;
-}
 
 // NG 16-head groups per workgroup (1 or 2; 4 NG waves): the groups share
 // the row tile and their dkv contributions are summed (chained MFMAs) before
@@ -129,6 +70,7 @@ __global__ void __launch_bounds__(256 * NG) sas_bwd_kernel(const BwdParams bp) {
   const int hw = hgw * 16 + h;                 // head in the workgroup
   const int hq = k.hg * NHD + hw;
   const int t = k.t;
+  if (bp.sparse_only && k.thr <= bp.dense_thr) return;   // sas_bwd_dq_kernel's token
   if (k.padded) {   // dq stays zero (the caller zeroes it)
     return;
   }
@@ -157,7 +99,8 @@ __global__ void __launch_bounds__(256 * NG) sas_bwd_kernel(const BwdParams bp) {
   const float delta = sum16(dpart);
   const float lse2 = p.lse[(size_t)t * p.H + hq] * kLog2e;
   if (part == 0) { lds_hd[hw][0] = delta; lds_hd[hw][1] = lse2; }
-  if (part == 0 && k.sp == 0) {
+  if (part == 0 && bp.sparse_only) bp.delta[(size_t)t * p.H + hq] = delta;
+  if (part == 0 && k.sp == 0 && !bp.sparse_only) {
     const float psink = __builtin_amdgcn_exp2f(p.sinks[hq] * kLog2e - lse2);
     atomicAdd(bp.d_sinks + hq, -psink * delta);
   }
@@ -307,13 +250,15 @@ __global__ void __launch_bounds__(256 * NG) sas_bwd_kernel(const BwdParams bp) {
   }
   // one split: the workgroup owns its heads' dq; several: each adds its share
   float* dqb = bp.dq + ((size_t)t * p.H + k.hg * NHD + hgw * 16 + 4 * g4) * D + c16;
+  QT* dqh = reinterpret_cast<QT*>(bp.dq) + ((size_t)t * p.H + k.hg * NHD + hgw * 16 + 4 * g4) * D + c16;
 #pragma unroll
   for (int j = 0; j < NDT; ++j) {
     const int ct = wl + 4 * j;
     if (ct >= D / 16) break;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      if (p.nsplit == 1) dqb[(size_t)i * D + ct * 16] = dqt[j][i];
+      if (bp.dq_direct) dqh[(size_t)i * D + ct * 16] = (QT)dqt[j][i];
+      else if (p.nsplit == 1) dqb[(size_t)i * D + ct * 16] = dqt[j][i];
       else atomicAdd(dqb + (size_t)i * D + ct * 16, dqt[j][i]);
     }
   }
@@ -367,6 +312,7 @@ __global__ void __launch_bounds__(512) sas_bwd64_kernel(const BwdParams bp) {
   const int g = wave >> 1, hh = wave & 1;
   const int c16 = lane & 15, g4 = lane >> 4;
   const int t = k.t, h0 = k.hg * NHD;
+  if (bp.sparse_only && k.thr <= bp.dense_thr) return;   // sas_bwd_dq_kernel's token
   if (k.padded) return;   // dq stays zero (the caller zeroes it)
 
   // Delta = dO . O: 8 threads per head, 64 channels each, 8-lane sums
@@ -386,7 +332,9 @@ __global__ void __launch_bounds__(512) sas_bwd64_kernel(const BwdParams bp) {
     if (part == 0) {
       lds_hd[hd][0] = dpart;
       lds_hd[hd][1] = lse2;
-      if (k.sp == 0) {
+      if (bp.sparse_only) {
+        bp.delta[(size_t)t * p.H + hq] = dpart;
+      } else if (k.sp == 0) {
         const float psink = __builtin_amdgcn_exp2f(p.sinks[hq] * kLog2e - lse2);
         atomicAdd(bp.d_sinks + hq, -psink * dpart);
       }
@@ -578,12 +526,14 @@ __global__ void __launch_bounds__(512) sas_bwd64_kernel(const BwdParams bp) {
   }
   // one split: the workgroup owns its heads' dq; several: each adds its share
   float* dqb = bp.dq + ((size_t)t * p.H + h0 + 16 * g + 4 * g4) * D + c16;
+  QT* dqh = reinterpret_cast<QT*>(bp.dq) + ((size_t)t * p.H + h0 + 16 * g + 4 * g4) * D + c16;
 #pragma unroll
   for (int j = 0; j < DQT; ++j) {
     const int ct = hh * DQT + j;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      if (p.nsplit == 1) dqb[(size_t)i * D + ct * 16] = dqt[j][i];
+      if (bp.dq_direct) dqh[(size_t)i * D + ct * 16] = (QT)dqt[j][i];
+      else if (p.nsplit == 1) dqb[(size_t)i * D + ct * 16] = dqt[j][i];
       else atomicAdd(dqb + (size_t)i * D + ct * 16, dqt[j][i]);
     }
   }
@@ -906,6 +856,58 @@ int launch_bwd_ng(const BwdParams& bp, int ng, int nblocks, hipStream_t st) {
   return ng == 2 ? launch_bwd<D, QT, 2>(bp, nblocks, st) : launch_bwd<D, QT, 1>(bp, nblocks, st);
 }
 
+// the per-token kernel over the whole call
+int launch_tokens(const BwdParams& bp, const SasFwdArgs* a, bool b64, int ng, int nblocks, hipStream_t st) {
+  if (b64) {
+    if (a->q_dtype == SAS_DT_BF16)
+      return a->D == 576 ? launch_bwd64<576, __bf16>(bp, nblocks, st) : launch_bwd64<512, __bf16>(bp, nblocks, st);
+    return a->D == 576 ? launch_bwd64<576, _Float16>(bp, nblocks, st) : launch_bwd64<512, _Float16>(bp, nblocks, st);
+  }
+  if (a->q_dtype == SAS_DT_BF16)
+    return a->D == 576 ? launch_bwd_ng<576, __bf16>(bp, ng, nblocks, st)
+                       : launch_bwd_ng<512, __bf16>(bp, ng, nblocks, st);
+  return a->D == 576 ? launch_bwd_ng<576, _Float16>(bp, ng, nblocks, st)
+                     : launch_bwd_ng<512, _Float16>(bp, ng, nblocks, st);
+}
+
+// The prefill path (sas_bwd_pre.hip): whether a call takes it, and its grid.
+// Query tokens share rows from about 64 tokens per batch on (as for the
+// window pass), and its head groups are 32 wide.
+#ifndef SAS_BWD_DENSE
+#define SAS_BWD_DENSE 8
+#endif
+struct PrePlan {
+  bool on, sparse;   // sparse: some tokens may need per-token adds for their compressed rows
+  int dense_thr;
+  long long seg_groups, cmp_tiles, win_tiles;
+  size_t ws;
+};
+PrePlan plan_prefill(const SasFwdArgs* a) {
+  PrePlan r{};
+  const long long nslots = (long long)a->win_left + 1 + (a->scenario >= SAS_CFA ? a->K : 0);
+  r.on = a->H % 32 == 0 && !(a->flags & SAS_BWD_WINDOW_TOKENS) && a->num_splits <= 0 &&
+         ((a->flags & SAS_BWD_WINDOW_KEYS) || a->T >= 64 * a->B);
+  if (!r.on) return r;
+  // A token with n compressed rows below its causal threshold and a list of K
+  // of them costs the key-major pass n row products (~0.2 ns each with 64
+  // heads when the chip is full) and the per-token kernel min(n, K) atomic
+  // adds per channel (1.77 ns): key-major up to n = 8 K.
+  const long long cap = a->scenario >= SAS_CFA ? a->cmp_bt_stride * a->cmp_block_size : 0;
+  const long long dense = a->scenario == SAS_SCFA ? std::min<long long>(INT_MAX, SAS_BWD_DENSE * a->K) : INT_MAX;
+  r.dense_thr = (int)dense;
+  r.sparse = a->scenario == SAS_SCFA && cap > dense;
+  const long long rows = a->scenario == SAS_CFA ? std::min<long long>(cap, a->K) : std::min(cap, dense);
+  r.seg_groups = a->T / kKeySeg + a->B;
+  r.cmp_tiles = (rows + kKeyRows - 1) / kKeyRows;
+  r.win_tiles = std::min<long long>(((long long)a->win_left + kKeySeg + 2 * (kKeyRows - 1)) / kKeyRows,
+                                    (a->ori_bt_stride * a->ori_block_size + kKeyRows - 1) / kKeyRows);
+  r.ws = (size_t)a->T * a->H * sizeof(float);
+  if ((r.sparse && nslots > kMaxSlots) || r.ws == 0 ||
+      (double)(r.cmp_tiles + r.win_tiles) * (r.seg_groups + 64) * (a->H / 32) > 2e9)
+    return PrePlan{};
+  return r;
+}
+
 }  // namespace
 }  // namespace sas
 
@@ -1017,6 +1019,12 @@ extern "C" int sas_bwd_v1(const SasBwdArgs* ba, void* stream) {
   // per-token adds there.
   if ((a->flags & SAS_BWD_WINDOW_TOKENS) && (a->flags & SAS_BWD_WINDOW_KEYS))
     return set_error(SAS_EINVAL, "bwd: SAS_BWD_WINDOW_TOKENS and SAS_BWD_WINDOW_KEYS together");
+  const bool direct = a->flags & SAS_BWD_DQ_DTYPE, have_ws = a->flags & SAS_BWD_WORKSPACE;
+  const PrePlan pre = plan_prefill(a);
+  if (direct && !(pre.on && have_ws))
+    return set_error(SAS_EINVAL, "bwd: SAS_BWD_DQ_DTYPE without SAS_BWD_WORKSPACE or where sas_bwd_plan does not allow it");
+  if (have_ws && pre.on && (!a->workspace || a->workspace_bytes < pre.ws))
+    return set_error(SAS_ENOWS, "bwd: workspace of %zu bytes required", pre.ws);
   bool capturing = false;
   {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -1025,6 +1033,27 @@ extern "C" int sas_bwd_v1(const SasBwdArgs* ba, void* stream) {
       cs = hipStreamCaptureStatusActive;   // unknown: as if capturing
     }
     capturing = cs != hipStreamCaptureStatusNone;
+  }
+  if (pre.on && have_ws && (direct || !capturing || (a->flags & SAS_BWD_WINDOW_KEYS))) {
+    bp.delta = (float*)a->workspace;
+    bp.dq_direct = direct;
+    bp.dense_thr = pre.dense_thr;
+    bp.npass = (int)((nslots + kMaxSlots - 1) / kMaxSlots);
+    bp.seg_groups = (int)pre.seg_groups;
+    bp.cmp_tiles = (int)pre.cmp_tiles;
+    bp.win_tiles_seg = (int)pre.win_tiles;
+    if (pre.sparse) {
+      // one split: every token's dq is written by one workgroup
+      BwdParams sb = bp;
+      sb.sparse_only = sb.win_pass = 1;
+      sb.f.nsplit = 1;
+      sb.f.slots_per_split = (int)nslots;
+      const int nb = (int)((a->T + fp.nxcd - 1) / fp.nxcd * fp.nhg * fp.nxcd);
+      const int rc = launch_tokens(sb, a, b64, ng, nb, (hipStream_t)stream);
+      if (rc) return rc;
+    }
+    fp.slots_per_split = (int)((nslots + bp.npass - 1) / bp.npass);
+    return launch_bwd_prefill(bp, (int)a->D, a->q_dtype, (hipStream_t)stream);
   }
   const bool win = (a->flags & SAS_BWD_WINDOW_KEYS) ||
                    (!(a->flags & SAS_BWD_WINDOW_TOKENS) && !capturing && a->T >= 64 * a->B);
@@ -1054,19 +1083,7 @@ extern "C" int sas_bwd_v1(const SasBwdArgs* ba, void* stream) {
       }
     }
   }
-  int rc;
-  if (b64) {
-    if (a->q_dtype == SAS_DT_BF16)
-      rc = a->D == 576 ? launch_bwd64<576, __bf16>(bp, nblocks, st) : launch_bwd64<512, __bf16>(bp, nblocks, st);
-    else
-      rc = a->D == 576 ? launch_bwd64<576, _Float16>(bp, nblocks, st) : launch_bwd64<512, _Float16>(bp, nblocks, st);
-  } else if (a->q_dtype == SAS_DT_BF16) {
-    rc = a->D == 576 ? launch_bwd_ng<576, __bf16>(bp, ng, nblocks, st)
-                     : launch_bwd_ng<512, __bf16>(bp, ng, nblocks, st);
-  } else {
-    rc = a->D == 576 ? launch_bwd_ng<576, _Float16>(bp, ng, nblocks, st)
-                     : launch_bwd_ng<512, _Float16>(bp, ng, nblocks, st);
-  }
+  int rc = launch_tokens(bp, a, b64, ng, nblocks, st);
   if (rc || !win || win_blocks == 0) return rc;
   hipStream_t wst = side ? side->st : st;
   if (a->q_dtype == SAS_DT_BF16)
@@ -1083,4 +1100,14 @@ extern "C" int sas_bwd_v1(const SasBwdArgs* ba, void* stream) {
     }
   }
   return rc;
+}
+
+extern "C" int sas_bwd_plan(const SasBwdArgs* ba, int32_t* dq_dtype, size_t* workspace_bytes) {
+  using namespace sas;
+  clear_error();
+  if (!ba) return set_error(SAS_EINVAL, "bwd: null args");
+  const PrePlan pre = ba->fwd.T >= 0 && ba->fwd.B >= 1 && ba->fwd.H >= 1 ? plan_prefill(&ba->fwd) : PrePlan{};
+  if (dq_dtype) *dq_dtype = pre.on;
+  if (workspace_bytes) *workspace_bytes = pre.ws;
+  return SAS_OK;
 }

@@ -101,7 +101,7 @@ constexpr int kRowPad = 64;
 static __shared__ uint64_t lds_rows[kMaxSlots + kRowPad];
 static __shared__ int lds_cnt[kRoundsMax][kMaxWaves];
 static __shared__ float lds_ml[kMaxWaves][2][16];
-static __shared__ int lds_tok[2];   // resolve(): the token's batch and padded flag
+static __shared__ int lds_tok[3];   // resolve(): the token's batch, padded flag and causal threshold
 // fp8 rows: the fp32 scale of each ring row's four 128-channel latent groups
 // ([group][ring row]; the ring holds the unscaled e4m3 values, exact in bf16)
 static __shared__ __attribute__((aligned(16))) float lds_fsc[4][kLdsRows];
@@ -239,6 +239,17 @@ __device__ __forceinline__ void dma16(const void* src, uint32_t lds_addr) {
       : "memory", "m0");
 }
 
+// dma16 from a wave-uniform base and a 32-bit lane offset
+__device__ __forceinline__ void dma16s(uint32_t off, const void* base, uint32_t lds_addr) {
+  asm volatile(
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %0, %1"
+      :
+      : "v"(off), "s"(base), "s"(lds_addr)
+      : "memory", "m0");
+}
+
 __device__ __forceinline__ uint32_t lds_addr_of(const void* p) {
   return (uint32_t)(uintptr_t)(const LDS_AS void*)p;
 }
@@ -365,6 +376,7 @@ __device__ __forceinline__ void merge_partials(const FwdParams& p, int t, int h0
 struct Tok {
   int t, hg, sp;     // token, head group, KV split
   int b, nvalid;     // batch, compacted row addresses in lds_rows
+  int thr;           // compressed rows below the token's causal position
   bool padded;       // (b, position) outside the batch's query length
 };
 
@@ -388,7 +400,7 @@ __device__ __forceinline__ Tok item_of(const FwdParams& p, int item) {
   k.t = item / per_tok;
   k.hg = (item % per_tok) / p.nsplit;
   k.sp = item % p.nsplit;
-  k.b = 0; k.nvalid = 0; k.padded = true;
+  k.b = 0; k.nvalid = 0; k.thr = 0; k.padded = true;
   return k;
 }
 
@@ -457,7 +469,7 @@ __device__ __forceinline__ void resolve(const FwdParams& p, Tok& k, int tid, int
     const int nwin = (padded || sg < 0) ? 0 : min(sg, p.win_left) + 1;
     const int wlo = sg - nwin + 1;                               // = max(sg - win_left, 0)
     const int thr = (padded || sg + 1 <= 0) ? 0 : (sg + 1) / p.cmp_ratio;
-    if (tid == 0) { lds_tok[0] = b; lds_tok[1] = padded; }
+    if (tid == 0) { lds_tok[0] = b; lds_tok[1] = padded; lds_tok[2] = thr; }
 
     // ---- round trip 2: block tables -----------------------------------------
     // Every table read is issued unconditionally at a clamped, in-range
@@ -529,6 +541,7 @@ __device__ __forceinline__ void resolve(const FwdParams& p, Tok& k, int tid, int
   }
   k.b = lds_tok[0];
   k.padded = lds_tok[1] != 0;
+  k.thr = lds_tok[2];
   __syncthreads();
   k.nvalid = nvalid;
 }

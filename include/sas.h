@@ -165,6 +165,14 @@ typedef struct SasFwdArgs {
    summation order. */
 #define SAS_BWD_WINDOW_TOKENS 2   /* per-token adds for window rows */
 #define SAS_BWD_WINDOW_KEYS 4     /* the key-major window pass */
+/* The prefill path of sas_bwd_v1: with SAS_BWD_WORKSPACE, fwd.workspace holds
+   the bytes sas_bwd_plan reports, and calls that would take the key-major
+   window pass sum the compressed rows' gradients key-major too, all on
+   `stream`. With SAS_BWD_DQ_DTYPE as well, where sas_bwd_plan allows it, dq is
+   [T, H, D] in the query dtype, written whole (it need not be zeroed), and the
+   path is taken under capture too. */
+#define SAS_BWD_WORKSPACE 8
+#define SAS_BWD_DQ_DTYPE 16
 
 /*
  * Split count the library would use (after auto-selection) and the
@@ -250,6 +258,11 @@ typedef struct SasBwdArgs {
 } SasBwdArgs;
 
 int sas_bwd_v1(const SasBwdArgs* a, void* stream);
+
+/* Whether these arguments may set SAS_BWD_DQ_DTYPE, and the workspace bytes of
+   SAS_BWD_WORKSPACE (0: none is used). Reads dims, scenario, num_splits and the
+   window flags only. */
+int sas_bwd_plan(const SasBwdArgs* a, int32_t* dq_dtype, size_t* workspace_bytes);
 
 /*
  * Paged-KV cache writer (no counterpart in the reference, whose tests build

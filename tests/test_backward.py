@@ -509,3 +509,42 @@ def test_gpu_backward_h48_d512_matches_oracle():
     dq, d_ori, d_cmp, d_snk = sparse_attn_sharedkv_backward(dout.cuda(), d.q, out, lse, **kw)
     torch.cuda.synchronize()
     _check_against_oracle("h48_d512", inp, dq, d_ori, d_cmp, d_snk, _oracle_bwd(inp, dout, out, lse))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,spec", [
+    # tokens on both sides of the density rule (8 K rows): dense ones by the
+    # key-major pass, the others by per-token adds; 64- and 32-head groups
+    ("both_h64", dict(B=1, H=64, q_lens=[400], kv_lens=[400], K=8)),
+    ("both_h32", dict(B=2, H=32, q_lens=[270, 90], kv_lens=[330, 500], K=8, D=512, bs=16)),
+    ("per_token_only", dict(B=1, H=64, q_lens=[100], kv_lens=[900], K=8, dtype=torch.float16)),
+    # a row listed twice counts twice
+    ("listed_twice", dict(B=1, H=64, q_lens=[200], kv_lens=[400], K=16,
+                          idx_fn=lambda i: torch.cat([i[..., :1], i[..., :-1]], -1))),
+    # more key slots than one resolution pass holds, and lists past 2048 entries
+    ("dense_passes", dict(B=1, H=64, q_lens=[70], kv_lens=[5200], K=0, scenario=2)),
+    ("long_lists", dict(B=1, H=128, q_lens=[66], kv_lens=[8600], K=2100, D=512, win=1)),
+    # segment and tile edges: 63, 64, 65 and 129 tokens, windows off the tile grid
+    ("edges", dict(B=4, H=32, q_lens=[63, 64, 65, 129], kv_lens=[63, 191, 65, 400], K=40, win=66, bs=16)),
+])
+def test_gpu_backward_prefill_path(name, spec):
+    """The prefill path's branches (dq in the query dtype from the call, fp32
+    from the prepared one), every gradient element against the oracle."""
+    from dsv4_amd.api import (prepare_sparse_attn_sharedkv_backward, sparse_attn_sharedkv,
+                              sparse_attn_sharedkv_backward)
+    from tests.test_gpu_parity import _small
+    inp = _small(**spec)
+    d = inp.to("cuda")
+    kw = d.api_kwargs()
+    out, lse = sparse_attn_sharedkv(d.q, return_softmax_lse=True, **kw)
+    g = torch.Generator().manual_seed(41)
+    dout = torch.randn(out.shape, generator=g).to(inp.q.dtype)
+    r = _oracle_bwd(inp, dout, out, lse)
+    got = sparse_attn_sharedkv_backward(dout.cuda(), d.q, out, lse, **kw)
+    pb = prepare_sparse_attn_sharedkv_backward(dout.cuda(), d.q, out, lse, **kw)
+    assert pb.dq.dtype == torch.float32
+    pb.launch()
+    torch.cuda.synchronize()
+    _check_against_oracle(name, inp, *got, r)
+    _check_against_oracle(f"{name} prepared", inp, *pb.result(), r)
+    assert torch.equal(pb.dq.to(got[0].dtype).cpu(), got[0].cpu())
