@@ -19,9 +19,9 @@
 // comes from its index list, counted into LDS.
 //
 // Forward + backward of a 4096-token, 64-head, top-k 512 step: 4.35 ms with
-// per-token adds (the window rows key-major beside them), 2.27 ms here (dq
-// 0.80, rows 1.14 ms); the backward of 2726 packed tokens with 128 heads 2.61
-// against 1.49 ms.
+// per-token adds (the window rows key-major beside them), 2.12 ms here (dq
+// 0.78, rows 1.11 ms); the backward of 2726 packed tokens with 128 heads 2.61
+// against 1.41 ms.
 
 #include "sas_bwd.h"
 
@@ -47,8 +47,9 @@ __global__ void __launch_bounds__(128 * NG) sas_bwd_dq_kernel(const BwdParams bp
   constexpr int KSH = D / 64;                 // S k-steps per channel half
   constexpr int VSH = kDV / 64;               // dP k-steps per channel half
   constexpr int DQT = D / 32;                 // dq tiles per wave
-  constexpr int NI = TR * CH / 64;            // DMA instructions per chunk
-  constexpr int OPS = (NI + NW - 1) / NW;
+  constexpr int RI = CH / 8;                  // DMA instructions per 8 rows (9 or 8)
+  constexpr int NP = 8 / NW;                  // of which a wave takes NP in each 8 rows
+  constexpr int OPS = 4 * NP + (RI == 9);     // and waves 0-3 one of the left-over ones
   constexpr int SG = kSwzGroup<CH>;
   constexpr int kRing = 2 * TR * CH;          // chunks
   constexpr int kX = NW * 4 * 64;             // exchange chunks
@@ -98,7 +99,25 @@ __global__ void __launch_bounds__(128 * NG) sas_bwd_dq_kernel(const BwdParams bp
   for (int j = 0; j < DQT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const float scale = p.scale_log2 / kLog2e;
   const int ksw = swz<CH>(c16);
+  // transposed reads: dq tile j at voff[j % TPG], whole swizzle groups apart
+  constexpr int TPG = SG / 2;
   const int vr = 4 * g4 + (c16 >> 2), vsw = swz<CH>(vr), vb = (c16 & 3) >> 1;
+  int voff[TPG];
+#pragma unroll
+  for (int q = 0; q < TPG; ++q) {
+    const int L = 2 * (hh * DQT + q) + vb;
+    voff[q] = (vr * CH + ((L & -SG) | ((L & (SG - 1)) ^ vsw))) * 16 + (c16 & 1) * 8;
+  }
+  // DMA: a chunk's layout repeats every 8 rows (RI instructions); the wave's
+  // lanes keep one (row, column) per instruction it takes of them
+  int prow[NP + 1];
+  uint32_t pcol[NP + 1];
+#pragma unroll
+  for (int i = 0; i <= NP; ++i) {
+    const int P = (i < NP ? wave + NW * i : 8) * 64 + lane, r = P / CH;
+    prow[i] = r;
+    pcol[i] = (uint32_t)((P - r * CH) ^ swz<CH>(r)) * 16;
+  }
 
   for (int pass = 0; pass < bp.npass; ++pass) {
     k.sp = pass;
@@ -112,31 +131,32 @@ __global__ void __launch_bounds__(128 * NG) sas_bwd_dq_kernel(const BwdParams bp
     if (nvalid == 0) continue;
     if (tid < kRowPad) lds_rows[nvalid + tid] = lds_rows[nvalid - 1];
     __syncthreads();
-    auto dma_rows = [&](int c) {
+    // chunk c's DMA instruction o, from row address ra (chunk nch reads the
+    // padding: the last row again); the next instruction's address is read
+    // behind it
+    auto row_addr = [&](int c, int o) {
       const uint32_t rb = __builtin_amdgcn_readfirstlane(lds_addr_of(lds_rows + c * TR));
-      const uint32_t kb = lds_addr_of(lds_b + (c & 1) * TR * CH);
-      uint64_t ra[OPS];
-#pragma unroll
-      for (int o = 0; o < OPS; ++o) {
-        const int P = (o * NW + wave) * 64 + lane, r = min(P / CH, TR - 1);
-        ra[o] = *reinterpret_cast<const LDS_AS uint64_t*>((size_t)(rb + 8u * (uint32_t)r));
-      }
-#pragma unroll
-      for (int o = 0; o < OPS; ++o) {
-        if (NI % NW && o * NW + wave >= NI) break;   // wave-uniform
-        const int P = (o * NW + wave) * 64 + lane, r = P / CH, c_ = P - r * CH;
-        dma16(reinterpret_cast<const void*>(ra[o] + (uint64_t)((c_ ^ swz<CH>(r)) * 16)),
-              __builtin_amdgcn_readfirstlane(kb + (o * NW + wave) * 64 * 16));
-      }
+      const int j = o < 4 * NP ? o & 3 : wave & 3;   // 8-row group
+      return *reinterpret_cast<const LDS_AS uint64_t*>((size_t)(rb + 8u * (uint32_t)(prow[o >> 2] + 8 * j)));
+    };
+    uint64_t ra;
+    auto dma_fire = [&](int c, int o) {
+      if (o == 4 * NP && wave >= 4) return;   // wave-uniform
+      const int j = o < 4 * NP ? o & 3 : wave & 3, m = o < 4 * NP ? wave + NW * (o >> 2) : 8;
+      dma16(reinterpret_cast<const void*>(ra + pcol[o >> 2]),
+            __builtin_amdgcn_readfirstlane(lds_addr_of(lds_b + (c & 1) * TR * CH) + (j * RI + m) * 1024));
+      if (o + 1 < OPS) ra = row_addr(c, o + 1);
     };
     const int nch = (nvalid + TR - 1) / TR;
-    dma_rows(0);
+    ra = row_addr(0, 0);
+#pragma unroll
+    for (int o = 0; o < OPS; ++o) dma_fire(0, o);
     for (int c = 0; c < nch; ++c) {
       const int nr = nvalid - c * TR;
       const uint4* kt = lds_b + (c & 1) * TR * CH;
       __builtin_amdgcn_s_waitcnt(0);   // known to the compiler: no wait of its own behind the DMA
       __builtin_amdgcn_s_barrier();
-      if (c + 1 < nch) dma_rows(c + 1);
+      ra = row_addr(c + 1, 0);
       // S^T and dP^T of the chunk's two 16-row tiles over this wave's channels
       f32x4 s[2], dp[2];
 #pragma unroll
@@ -166,14 +186,12 @@ __global__ void __launch_bounds__(128 * NG) sas_bwd_dq_kernel(const BwdParams bp
             dp[0] = mfma32k<QT>(a0, of[i], dp[0]);
             dp[1] = mfma32k<QT>(a1, of[i], dp[1]);
           }
+          // the next chunk's DMA between the MFMAs (see sas_bwd_keys_kernel)
+          constexpr int EV = OPS > 5 ? 1 : 2;
+          if (i % EV == EV - 1 && i / EV < OPS) dma_fire(c + 1, i / EV);
         }
-        __builtin_amdgcn_sched_group_barrier(0x100, 2 * PF, HH);
 #pragma unroll
-        for (int i = 0; i < NF; ++i) {
-          if (i >= OFF) __builtin_amdgcn_sched_group_barrier(0x008, 2, HH);
-          if (i < VSH) __builtin_amdgcn_sched_group_barrier(0x008, 2, HH);
-          if (i + PF < NF) __builtin_amdgcn_sched_group_barrier(0x100, 2, HH);
-        }
+        for (int o = NF / (OPS > 5 ? 1 : 2); o < OPS; ++o) dma_fire(c + 1, o);
       };
       if (hh) half(std::integral_constant<int, 1>{});
       else half(std::integral_constant<int, 0>{});
@@ -200,9 +218,7 @@ __global__ void __launch_bounds__(128 * NG) sas_bwd_dq_kernel(const BwdParams bp
       const uint4 bds = make_uint4(pk[0], pk[1], pk[2], pk[3]);
       // dq^T: A = K^T of keys 4 g4 .. + 3 and 16 + 4 g4 .. + 3, the order of bds
       auto vfrag = [&](int j) {
-        const int L = 2 * (hh * DQT + j) + vb;
-        const uint4* a0 = kt + vr * CH + ((L & -SG) | ((L & (SG - 1)) ^ vsw));
-        const char* b0 = reinterpret_cast<const char*>(a0) + (c16 & 1) * 8;
+        const char* b0 = reinterpret_cast<const char*>(kt) + voff[j % TPG] + (j / TPG) * SG * 16;
         const uint2 u0 = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS i16x4*)(b0)));
         const uint2 u1 = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS i16x4*)(b0 + 16 * CH * 16)));
         return make_uint4(u0.x, u0.y, u1.x, u1.y);
@@ -224,6 +240,7 @@ __global__ void __launch_bounds__(128 * NG) sas_bwd_dq_kernel(const BwdParams bp
         if (j + PV < DQT) __builtin_amdgcn_sched_group_barrier(0x100, 2, 2);
       }
     }
+    wait_vm<0>();      // the spare chunk's DMA
     __syncthreads();   // the row list and the slots are free
   }
   // lane (g4, c16): channels 16 ct + 4 g4 .. + 3 of head c16
@@ -376,32 +393,40 @@ __global__ void __launch_bounds__(512) sas_bwd_keys_kernel(const BwdParams bp) {
   // registers and put into LDS one unit ahead; its q and dO one unit ahead by
   // DMA.
   const bool list = cmp && p.scenario == SAS_SCFA;
-  const bool list_reg = p.K <= kIdx * 512;
+  const int nidx = list ? (p.K + 511) >> 9 : 0;   // entries per thread
+  const bool list_reg = nidx <= kIdx;
   float hv = 0.f;
   int iv[kIdx];
+#pragma unroll
+  for (int i = 0; i < kIdx; ++i) iv[i] = -1;
   auto load_small = [&](int a) {
     const size_t t = (size_t)qp + a;
-    if (tid < 64) hv = tid < 32 ? p.lse[t * p.H + h0 + tid] : bp.delta[t * p.H + h0 + tid - 32];
-    if (list && list_reg) {
+    if (wave == 0) hv = (lane < 32 ? p.lse : bp.delta)[t * p.H + h0 + (lane & 31)];
+    if (list_reg) {
+      const int32_t* ix = p.cmp_idx + t * p.K;
 #pragma unroll
       for (int i = 0; i < kIdx; ++i) {
-        iv[i] = -1;
-        if (i * 512 < p.K && i * 512 + tid < p.K) iv[i] = p.cmp_idx[t * p.K + i * 512 + tid];
+        if (i >= nidx) break;   // uniform
+        iv[i] = ix[min(i * 512 + tid, p.K - 1)];
       }
     }
   };
   auto put_small = [&](int a, int buf) {
-    if (tid < 64) lds_h[buf][tid >> 5][tid & 31] = tid < 32 ? hv * kLog2e : hv;
+    if (wave == 0) lds_h[buf][lane >> 5][lane & 31] = lane < 32 ? hv * kLog2e : hv;
     if (list) {
-      const int thr = (sg0 + a + 1) / p.cmp_ratio;
-      auto put = [&](int i) {
-        if (i >= p0 && i < p0 + kKeyRows && i < thr) atomicAdd(&lds_c[buf][i - p0], 1);
-      };
+      const unsigned top = (unsigned)min((sg0 + a + 1) / p.cmp_ratio - p0, kKeyRows);   // >= 1: rows below the threshold
       if (list_reg) {
 #pragma unroll
-        for (int i = 0; i < kIdx; ++i) put(iv[i]);
+        for (int i = 0; i < kIdx; ++i) {
+          if (i >= nidx) break;   // uniform
+          const unsigned r = (unsigned)(iv[i] - p0);
+          if (r < top && i * 512 + tid < p.K) atomicAdd(&lds_c[buf][r], 1);
+        }
       } else {
-        for (int i = tid; i < p.K; i += 512) put(p.cmp_idx[((size_t)qp + a) * p.K + i]);
+        for (int i = tid; i < p.K; i += 512) {
+          const unsigned r = (unsigned)(p.cmp_idx[((size_t)qp + a) * p.K + i] - p0);
+          if (r < top) atomicAdd(&lds_c[buf][r], 1);
+        }
       }
     }
   };
@@ -414,17 +439,15 @@ __global__ void __launch_bounds__(512) sas_bwd_keys_kernel(const BwdParams bp) {
   const uint32_t oq = (uint32_t)(rq * CH + ((Pq - rq * CH) ^ swz<CH>(rq))) * 16;
   const uint32_t ox = (uint32_t)(rx * CH + ((Px - rx * CH) ^ swz<CH>(rx))) * 16;
   const uint32_t oo = (uint32_t)(wave * OCH + (lane ^ swz<OCH>(wave))) * 16;
-  auto dma = [&](int a, int buf) {
+  auto dma = [&](int a, int buf, int i) {   // instruction i < 9 of the wave
     const size_t t = (size_t)qp + a;
     const uint8_t* qs = p.q + (t * p.H + h0) * D * 2;
     const uint8_t* os = bp.dout + (t * p.H + h0) * kDV * 2;
     const uint32_t qb = lds_addr_of(lds_q[buf]) + wave * 1024, ob = lds_addr_of(lds_o[buf]) + wave * 1024;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      dma16s(oq, qs + j * 8 * D * 2, __builtin_amdgcn_readfirstlane(qb + j * RI * 1024));
-      dma16s(oo, os + j * 8 * kDV * 2, __builtin_amdgcn_readfirstlane(ob + j * 8 * 1024));
-    }
-    if (RI == 9 && wave < 4)
+    const int j = i >> 1;
+    if (i < 8 && !(i & 1)) dma16s(oq, qs + j * 8 * D * 2, __builtin_amdgcn_readfirstlane(qb + j * RI * 1024));
+    if (i < 8 && (i & 1)) dma16s(oo, os + j * 8 * kDV * 2, __builtin_amdgcn_readfirstlane(ob + j * 8 * 1024));
+    if (i == 8 && RI == 9 && wave < 4)
       dma16s(ox, qs + wave * 8 * D * 2, __builtin_amdgcn_readfirstlane(lds_addr_of(lds_q[buf]) + (8 + 9 * wave) * 1024));
   };
 
@@ -458,7 +481,8 @@ __global__ void __launch_bounds__(512) sas_bwd_keys_kernel(const BwdParams bp) {
   load_small(a0);
   put_small(a0, 0);
   load_small(min(a0 + 1, a1 - 1));
-  dma(a0, 0);
+#pragma unroll
+  for (int i = 0; i < 9; ++i) dma(a0, 0, i);
   for (int a = a0; a < a1; ++a) {
     const int buf = (a - a0) & 1;
     // the builtin, not asm: every load the compiler tracks (the rows, the
@@ -466,11 +490,8 @@ __global__ void __launch_bounds__(512) sas_bwd_keys_kernel(const BwdParams bp) {
     // its own behind the DMA issued below
     __builtin_amdgcn_s_waitcnt(0);
     __builtin_amdgcn_s_barrier();
-    if (a + 1 < a1) {   // uniform
-      put_small(a + 1, buf ^ 1);
-      load_small(min(a + 2, a1 - 1));
-      dma(a + 1, buf ^ 1);
-    }
+    // (past the last unit it is staged again, into the spare buffer)
+    const int an = min(a + 1, a1 - 1);
     const uint4* tq = lds_q[buf];
     const uint4* to = lds_o[buf];
     {
@@ -494,6 +515,8 @@ __global__ void __launch_bounds__(512) sas_bwd_keys_kernel(const BwdParams bp) {
       uint4 qa[PF], oa[PF];
 #pragma unroll
       for (int i = 0; i < PF; ++i) { qa[i] = qfrag(kq(i)); oa[i] = ofrag(ko(i)); }
+      put_small(an, buf ^ 1);
+      load_small(min(a + 2, a1 - 1));
 #pragma unroll
       for (int i = 0; i < KS; ++i) {
         const uint4 qv = qa[i % PF];
@@ -504,14 +527,12 @@ __global__ void __launch_bounds__(512) sas_bwd_keys_kernel(const BwdParams bp) {
           if (i + PF < VS) oa[i % PF] = ofrag(ko(i + PF));
           dc[i & 1] = mfma32k<QT>(ov, kf[ko(i)], dc[i & 1]);
         }
-      }
-      // the reads PF fragments ahead, one behind each MFMA (the scheduler's
-      // own order reads each fragment right before its MFMA)
-      __builtin_amdgcn_sched_group_barrier(0x100, 2 * PF + 3, 0);
-#pragma unroll
-      for (int i = 0; i < KS + VS; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        if (i < KS + VS - 2 * PF) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        // the next unit's DMA, an instruction every few MFMAs: issued at once
+        // they fill the CU's memory pipeline and hold every wave ahead of its
+        // MFMAs (unit 6100 clk against 4900; in the dkv phase instead they
+        // land too late). The asm also keeps the reads PF fragments ahead,
+        // where the scheduler would sink each one to its MFMA.
+        if (i % 2 == 1) dma(an, buf ^ 1, i / 2);
       }
       const f32x4 s_ = sc[0] + sc[1], d_ = dc[0] + dc[1];
       // lane (g4, c16): heads 16 ht + 4 g4 .. + 3 of row 16 rt + c16
@@ -573,6 +594,7 @@ __global__ void __launch_bounds__(512) sas_bwd_keys_kernel(const BwdParams bp) {
       if (ROPE) __builtin_amdgcn_sched_group_barrier(0x008, 2, 1);
     }
   }
+  wait_vm<0>();   // the spare unit's DMA
   // lane (g4, c16): rows 16 r + 4 g4 + i, channel 16 ct + c16
   const uint64_t lo = reinterpret_cast<uint64_t>(cmp ? p.cmp_kv : p.ori_kv);
   float* db = cmp ? bp.d_cmp : bp.d_ori;
