@@ -39,7 +39,7 @@
 // decode), :628-722 (window / compressed masks), :594-617 (sink seed),
 // :877 (P cast), :1135-1145 (LSE), and golden.py:69-204.
 
-#include "sas_kern.h"
+#include "sas_fwd_win.h"
 
 #include <mutex>
 
@@ -2072,6 +2072,17 @@ int make_plan(const SasFwdArgs* a, Plan* pl) {
   return SAS_OK;
 }
 
+// Window-only calls walk runs of tokens (sas_fwd_win.hip) once one workgroup
+// per (token, head group) would take more than one round of the CUs. Below
+// that the run's first window costs more than it saves (64 heads, D = 576:
+// 128 tokens 15.2 against 14.4 us, 256 tokens 17.3 against 16.2, 384 tokens
+// 21.6 against 27.4, 1000 tokens 39 against 55; 16 heads, 1500 tokens 22
+// against 66).
+bool win_runs(const SasFwdArgs* a, const Plan& pl) {
+  return pl.exact && a->scenario == SAS_SWA && a->kv_dtype == a->q_dtype && a->win_left < 128 &&
+         a->head_waves == 0 && (long long)a->T * pl.nhg > sas::device_cus();
+}
+
 template <int HW, int NW, int D, typename QT, int KVF, bool EXW = false>
 int launch_fwd(const FwdParams& fp, int nblocks, hipStream_t st) {
   hipLaunchKernelGGL((sas_fwd_kernel<HW, NW, D, QT, KVF, EXW>), dim3(nblocks), dim3(NW * 64), 0, st, fp);
@@ -2226,6 +2237,10 @@ extern "C" int sas_fwd_v1(const SasFwdArgs* a, void* stream) {
   fp.out_nt = pl.nsplit == 1 && (size_t)a->T * a->H * kDV * 2 >= (size_t(16) << 20);
   hipStream_t st = (hipStream_t)stream;
 
+  if (win_runs(a, pl)) {
+    const int cus = sas::device_cus();
+    return launch_fwd_win(fp, (int)a->D, a->q_dtype, (int)std::min<long long>(64, (a->T + cus - 1) / cus), st);
+  }
   if (fp8) rc = dispatch_hw<576, __bf16, 1>(pl.hw, pl.nw, pl.exact, fp, nblocks, st);
   else if (a->q_dtype == SAS_DT_BF16)
     rc = a->D == 576 ? dispatch_hw<576, __bf16, 0>(pl.hw, pl.nw, pl.exact, fp, nblocks, st)

@@ -777,3 +777,62 @@ def test_fp8_dequant_bit_exact_through_one_row_windows(H, scenario, waves):
     for h in range(H):   # by value: code 0x80 (-0.0) accumulates to +0.0
         assert torch.equal(got[:, h].float(), want.float()), \
             f"head {h}: {int((got[:, h].float() != want.float()).sum())} channels differ"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,spec", [
+    # more tokens than one round of workgroups; runs, groups and ring wraps
+    ("h64", dict(B=1, H=64, q_lens=[700], kv_lens=[700])),
+    ("h64_d512", dict(B=2, H=64, q_lens=[333, 260], kv_lens=[1333, 300], D=512, bs=16)),
+    ("h128_fp16", dict(B=3, H=128, q_lens=[1, 170, 129], kv_lens=[900, 171, 129], dtype=torch.float16)),
+    ("h48_win64", dict(B=2, H=48, q_lens=[300, 301], kv_lens=[310, 2000], win=63)),
+    ("h16_win1", dict(B=1, H=16, q_lens=[1100], kv_lens=[1100], win=0, D=512)),
+    # queries longer than the cache: the first tokens attend the sink only
+    ("short_kv", dict(B=2, H=64, q_lens=[300, 200], kv_lens=[120, 3], win=126)),
+    ("missing_blocks", dict(B=1, H=64, q_lens=[600], kv_lens=[900], bs=16)),
+])
+def test_window_runs_match_per_token(name, spec):
+    """Window-only prefills by runs of tokens against the one-workgroup-per-
+    token kernel (head_waves given), whose parity the tests above hold: the
+    scores differ by fp32 summation order, which moves a P by at most one
+    rounding step (2^-8 in bf16, 2^-11 in fp16) of its value."""
+    from dsv4_amd.api import prepare_sparse_attn_sharedkv
+    inp = _small(K=0, scenario=1, **spec)
+    if name == "missing_blocks":
+        inp.ori_bt[0, 3::5] = -1
+    d = inp.to("cuda")
+    kw = d.api_kwargs()
+    res = []
+    for hw in (0, 1):
+        pc = prepare_sparse_attn_sharedkv(d.q, head_waves=hw, **kw)
+        pc.out.fill_(float("nan"))
+        pc.launch()
+        torch.cuda.synchronize()
+        res.append((pc.out.float().cpu(), pc.lse.cpu()))
+    (o0, l0), (o1, l1) = res
+    step = 2.0 ** -8 if inp.q.dtype == torch.bfloat16 else 2.0 ** -11
+    assert torch.isfinite(o0).all()
+    torch.testing.assert_close(l0, l1, atol=2e-5, rtol=2e-6)
+    # |dO| <= step sum_j p_j |v_j| + the output's own rounding
+    vmax = float(inp.ori_kv.abs().max())
+    assert float((o0 - o1).abs().max()) <= step * vmax
+    assert float((o0 - o1).norm() / o1.norm().clamp_min(1e-9)) < step
+
+
+@pytest.mark.gpu
+def test_window_runs_bsnd_padding():
+    """Padded query rows (per-batch lengths below S) give zeros, the others
+    the packed call's values."""
+    from dsv4_amd.api import sparse_attn_sharedkv
+    lens = [300, 170]
+    inp = _small(B=2, H=64, q_lens=lens, kv_lens=[400, 170], K=0, scenario=1)
+    d = inp.to("cuda")
+    kw = d.api_kwargs()
+    ref, lref = sparse_attn_sharedkv(d.q, return_softmax_lse=True, **kw)
+    q = torch.randn(2, 300, 64, 576).to(torch.bfloat16).cuda()
+    q[0], q[1, :170] = d.q[:300], d.q[300:]
+    out, lse = sparse_attn_sharedkv(q, return_softmax_lse=True, **dict(kw, layout_q="BSND"))
+    torch.cuda.synchronize()
+    assert torch.equal(out[0], ref[:300]) and torch.equal(out[1, :170], ref[300:])
+    assert torch.equal(lse[0], lref[:300]) and torch.equal(lse[1, :170], lref[300:])
+    assert torch.count_nonzero(out[1, 170:]) == 0 and torch.count_nonzero(lse[1, 170:]) == 0
