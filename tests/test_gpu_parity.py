@@ -836,3 +836,42 @@ def test_window_runs_bsnd_padding():
     assert torch.equal(out[0], ref[:300]) and torch.equal(out[1, :170], ref[300:])
     assert torch.equal(lse[0], lref[:300]) and torch.equal(lse[1, :170], lref[300:])
     assert torch.count_nonzero(out[1, 170:]) == 0 and torch.count_nonzero(lse[1, 170:]) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,spec", [
+    ("h64", dict(B=1, H=64, q_lens=[1100], kv_lens=[1100], ratio=16)),
+    ("h128_d512_fp16", dict(B=2, H=128, q_lens=[400, 130], kv_lens=[3400, 130], ratio=32, D=512, bs=16, dtype=torch.float16)),
+    # the limits of the run's tables (128 window rows + runs, 128 compressed), a compressed row per token
+    ("limits", dict(B=1, H=64, q_lens=[1030], kv_lens=[1031], ratio=8, D=512, win=128)),
+    ("ratio1_win1", dict(B=9, H=64, q_lens=[128] * 9, kv_lens=[128] * 9, ratio=1, win=0)),
+    ("short_kv", dict(B=2, H=64, q_lens=[800, 300], kv_lens=[350, 3], ratio=4, win=40)),
+    ("missing_blocks", dict(B=1, H=64, q_lens=[1050], kv_lens=[1050], ratio=16, bs=16)),
+])
+def test_dense_runs_match_per_token(name, spec):
+    """Dense compressed prefills by runs of tokens against the one-workgroup-
+    per-token kernel (head_waves given). The two round P against different
+    running maxima: each key's weight differs by at most a rounding step of
+    each (2 x 2^-9 relative in bf16, 2 x 2^-12 in fp16), and the output rounds
+    once more."""
+    from dsv4_amd.api import prepare_sparse_attn_sharedkv
+    inp = _small(K=0, scenario=2, **spec)
+    if name == "missing_blocks":
+        inp.ori_bt[0, 3::5] = -1
+        inp.cmp_bt[0, 1] = -1
+    d = inp.to("cuda")
+    kw = d.api_kwargs()
+    res = []
+    for hw in (0, 4):
+        pc = prepare_sparse_attn_sharedkv(d.q, head_waves=hw, **kw)
+        pc.out.fill_(float("nan"))
+        pc.launch()
+        torch.cuda.synchronize()
+        res.append((pc.out.float().cpu(), pc.lse.cpu()))
+    (o0, l0), (o1, l1) = res
+    step = 2.0 ** -8 if inp.q.dtype == torch.bfloat16 else 2.0 ** -11
+    assert torch.isfinite(o0).all()
+    torch.testing.assert_close(l0, l1, atol=2e-5, rtol=2e-6)
+    vmax = float(max(inp.ori_kv.abs().max(), inp.cmp_kv.abs().max()))
+    assert float((o0 - o1).abs().max()) <= 2 * step * vmax
+    assert float((o0 - o1).norm() / o1.norm().clamp_min(1e-9)) < step
