@@ -19,16 +19,17 @@ need it for scheduling: it launches one workgroup per (token, head group,
 KV split) and covers every valid token by construction; an omitted one is
 built with the bit-exact scheduler on request (:meth:`PreparedCall.metadata`).
 
-Host cost of a call: the argument resolution (routing, checks, launch
-arguments, split plan) is cached per call signature (shapes, dtypes, device
-pointers, scalars, stream), so a repeated call allocates ``out`` / ``lse``,
-copies host-side sequence lengths through a reused pinned buffer, and
-launches. Device ``cu_seqlens_q`` is passed to the kernel as it is.
+Host cost of a call: the argument resolution (routing, checks, split plan) is
+cached per call signature (shapes, dtypes, devices, scalars), so a call of a
+shape seen before, on whatever buffers, allocates ``out`` / ``lse``, copies
+host-side sequence lengths through a reused pinned buffer, and launches.
+Device ``cu_seqlens_q`` is passed to the kernel as it is.
 """
 
 from __future__ import annotations
 
 import ctypes as C
+import struct
 import threading
 from collections import OrderedDict
 from typing import Optional, Tuple, Union
@@ -618,19 +619,28 @@ def prepare_sparse_attn_sharedkv(
 # ---------------------------------------------------------------------------
 
 _CACHE_MAX = 64
-_cache: "OrderedDict[tuple, _Resolved]" = OrderedDict()
+_cache: "OrderedDict[tuple, _Cached]" = OrderedDict()
 _cache_lock = threading.Lock()
 
 
-def _sig(t):
-    """What a launch depends on for a tensor: device tensors by address and
-    geometry (their values are read by the kernel), host tensors by geometry
-    (their values are copied per call)."""
-    if t is None:
-        return None
-    if t.is_cuda:
-        return (t.data_ptr(), t.shape, t.stride(), t.dtype, t.device.index)
-    return ("host", t.shape, t.dtype)
+# SasFwdArgs starts with its pointers (q, ori_kv, ori_block_table, cmp_kv,
+# cmp_block_table, cmp_indices, q_prefix, act_q, act_kv, sinks, out, lse,
+# workspace) and workspace_bytes; the rest of a call's arguments (dims, strides,
+# the plan) follows from its signature and is kept as bytes behind them.
+_PTRS = struct.Struct("@14Q")
+assert _lib.SasFwdArgs.T.offset == _PTRS.size
+_fwd_raw = None
+
+
+def _fwd_bytes():
+    """sas_fwd_v1 taking its arguments as packed bytes."""
+    global _fwd_raw
+    if _fwd_raw is None:
+        f = _lib.lib()["sas_fwd_v1"]   # a function object of its own: other argument types
+        f.argtypes = [C.c_char_p, C.c_void_p]
+        f.restype = C.c_int
+        _fwd_raw = f
+    return _fwd_raw
 
 
 def sparse_attn_sharedkv(
@@ -665,36 +675,51 @@ def sparse_attn_sharedkv(
     (BSND) in q's dtype; ``lse`` is fp32 ``[T1, N1]`` / ``[B, S1, N1]`` with
     ``lse = max + ln(sum)`` over all attended keys and the sink.
     """
-    dev = q.device
-    stream = _raw_stream(dev) if q.is_cuda else None
     # CFA's slot count follows the longest sequence (api.py:259-261): part of
     # the signature, read from the host copy, or through a sync as the
     # reference does for device lengths
     cfa_k = None
     if cmp_kv is not None and cmp_sparse_indices is None and seqused_kv.numel():
         cfa_k = int(seqused_kv.max().item())
-    key = (_sig(q), _sig(ori_kv), _sig(cmp_kv), _sig(cmp_sparse_indices), _sig(ori_block_table),
-           _sig(cmp_block_table), _sig(cu_seqlens_q), _sig(seqused_kv), _sig(sinks),
+    # The signature is the tensors' geometry: what a resolution holds (checks,
+    # dims, the split plan) depends on no address, so new buffers of a shape
+    # seen before pay nothing extra. (With the addresses in it, and 9 helper
+    # calls to build it, a repeated 1-token call took the host 13.5 us and the
+    # first on new buffers 96 us.)
+    key = (q.shape, q.dtype, q.get_device(), q.is_contiguous(),
+           ori_kv.shape, ori_kv.dtype, ori_kv.get_device(), ori_kv.is_contiguous(),
+           ori_block_table.shape, ori_block_table.dtype, ori_block_table.get_device(), ori_block_table.is_contiguous(),
+           seqused_kv.shape, seqused_kv.dtype, seqused_kv.get_device(), seqused_kv.is_contiguous(),
+           sinks.shape, sinks.dtype, sinks.get_device(), sinks.is_contiguous(),
+           None if cu_seqlens_q is None else
+           (cu_seqlens_q.shape, cu_seqlens_q.dtype, cu_seqlens_q.get_device(), cu_seqlens_q.is_contiguous()),
+           None if cmp_kv is None else (cmp_kv.shape, cmp_kv.dtype, cmp_kv.get_device(), cmp_kv.is_contiguous()),
+           None if cmp_block_table is None else
+           (cmp_block_table.shape, cmp_block_table.dtype, cmp_block_table.get_device(), cmp_block_table.is_contiguous()),
+           None if cmp_sparse_indices is None else
+           (cmp_sparse_indices.shape, cmp_sparse_indices.dtype, cmp_sparse_indices.get_device(),
+            cmp_sparse_indices.is_contiguous()),
            None if metadata is None else metadata.numel(), float(softmax_scale), cmp_ratio, ori_mask_mode,
-           cmp_mask_mode, ori_win_left, ori_win_right, layout_q, layout_kv, core_num, topk_cmp, cfa_k, stream)
-    with _cache_lock:
-        r = _cache.get(key)
-        if r is not None:
-            _cache.move_to_end(key)
-    hit = r is not None
-    if not hit:
-        r = _resolve(q, ori_kv=ori_kv, cmp_kv=cmp_kv, cmp_sparse_indices=cmp_sparse_indices,
-                     ori_block_table=ori_block_table, cmp_block_table=cmp_block_table,
-                     cu_seqlens_q=cu_seqlens_q, seqused_q=seqused_q, seqused_kv=seqused_kv, sinks=sinks,
-                     metadata=metadata, softmax_scale=softmax_scale, cmp_ratio=cmp_ratio,
-                     ori_mask_mode=ori_mask_mode, cmp_mask_mode=cmp_mask_mode, ori_win_left=ori_win_left,
-                     ori_win_right=ori_win_right, layout_q=layout_q, layout_kv=layout_kv,
-                     core_num=core_num, topk_cmp=topk_cmp, num_splits=0, head_waves=0, waves=0)
-        if r.cacheable:
-            with _cache_lock:
-                _cache[key] = r
-                if len(_cache) > _CACHE_MAX:
-                    _cache.popitem(last=False)
+           cmp_mask_mode, ori_win_left, ori_win_right, layout_q, layout_kv, core_num, topk_cmp, cfa_k)
+    r = _cache.get(key)
+    dev = q.device
+    stream = _raw_stream(dev) if q.is_cuda else None
+    if r is not None:
+        return _run_cached(r, stream, dev, q, ori_kv, cmp_kv, cmp_sparse_indices, ori_block_table, cmp_block_table,
+                           cu_seqlens_q, seqused_kv, sinks, return_softmax_lse)
+    r = _resolve(q, ori_kv=ori_kv, cmp_kv=cmp_kv, cmp_sparse_indices=cmp_sparse_indices,
+                 ori_block_table=ori_block_table, cmp_block_table=cmp_block_table,
+                 cu_seqlens_q=cu_seqlens_q, seqused_q=seqused_q, seqused_kv=seqused_kv, sinks=sinks,
+                 metadata=metadata, softmax_scale=softmax_scale, cmp_ratio=cmp_ratio,
+                 ori_mask_mode=ori_mask_mode, cmp_mask_mode=cmp_mask_mode, ori_win_left=ori_win_left,
+                 ori_win_right=ori_win_right, layout_q=layout_q, layout_kv=layout_kv,
+                 core_num=core_num, topk_cmp=topk_cmp, num_splits=0, head_waves=0, waves=0)
+    if r.cacheable:
+        kept = _Cached(r)
+        with _cache_lock:
+            _cache[key] = kept
+            if len(_cache) > _CACHE_MAX:
+                _cache.popitem(last=False)
     out = torch.empty((r.T1, r.N1, 512), dtype=r.dtype, device=dev)
     lse = torch.empty((r.T1, r.N1), dtype=torch.float32, device=dev)
     a = _lib.SasFwdArgs.from_buffer_copy(r.args)
@@ -702,19 +727,13 @@ def sparse_attn_sharedkv(
     keep = []
     staged = None
     if r.host_parts:
-        parts = r.host_parts
-        if hit:
-            # this call's host lengths (a cached resolution, TND only, holds
-            # an earlier call's)
-            cur = {"cu": cu_seqlens_q, "kv": seqused_kv}
-            parts = [(name, _host_i32(cur[name])) for name, _ in r.host_parts]
         if not torch.cuda.is_current_stream_capturing():
             ring = _seqlen_ring(dev)
-            staged = ring.stage([(t.data_ptr(), t.numel()) for _, t in parts], stream)
+            staged = ring.stage([(t.data_ptr(), t.numel()) for _, t in r.host_parts], stream)
         if staged is not None:
-            _point_seqlens(parts, a, staged[0])
+            _point_seqlens(r.host_parts, a, staged[0])
         else:
-            _bind_seqlens(r, parts, a, torch.cuda.current_stream(dev), keep)
+            _bind_seqlens(r, r.host_parts, a, torch.cuda.current_stream(dev), keep)
     try:
         if r.ws_bytes:
             ws = _workspace(dev, stream, r.ws_bytes)
@@ -724,6 +743,59 @@ def sparse_attn_sharedkv(
         if staged is not None:
             ring.release(staged[1], stream)
     return _result(out, lse, r.layout_q, r.B, r.S_max, return_softmax_lse)
+
+
+class _Cached:
+    """What a signature's later calls need of its resolution: no tensor, no
+    address (TND calls whose operands are used as given)."""
+
+    __slots__ = ("out_shape", "lse_shape", "tail", "ws_bytes", "host_names", "B")
+
+    def __init__(self, r: _Resolved):
+        self.out_shape, self.lse_shape = (r.T1, r.N1, 512), (r.T1, r.N1)
+        self.tail = bytes(r.args)[_PTRS.size:]
+        self.ws_bytes = r.ws_bytes
+        self.host_names = [name for name, _ in r.host_parts]
+        self.B = r.B
+
+
+def _run_cached(r: _Cached, stream, dev, q, ori_kv, cmp_kv, cmp_sparse_indices, ori_block_table, cmp_block_table,
+                cu_seqlens_q, seqused_kv, sinks, return_softmax_lse):
+    out = q.new_empty(r.out_shape)
+    lse = sinks.new_empty(r.lse_shape)   # fp32 on the device, or the call would not be cached
+    cu, kv = cu_seqlens_q.data_ptr(), seqused_kv.data_ptr()
+    keep = staged = None
+    if r.host_names:
+        cur = {"cu": cu_seqlens_q, "kv": seqused_kv}
+        parts = [_host_i32(cur[name]) for name in r.host_names]
+        if not torch.cuda.is_current_stream_capturing():
+            ring = _seqlen_ring(dev)
+            staged = ring.stage([(t.data_ptr(), t.numel()) for t in parts], stream)
+        if staged is not None:
+            base = staged[0]
+        else:
+            keep = _stage(parts, dev, torch.cuda.current_stream(dev))
+            base = keep.data_ptr()
+        for name, t in zip(r.host_names, parts):
+            if name == "cu":
+                cu = base
+            else:
+                kv = base
+            base += 4 * t.numel()
+    try:
+        ws = _workspace(dev, stream, r.ws_bytes).data_ptr() if r.ws_bytes else 0
+        cmp_ = cmp_kv is not None
+        rc = _fwd_bytes()(
+            _PTRS.pack(q.data_ptr(), ori_kv.data_ptr(), ori_block_table.data_ptr(), cmp_kv.data_ptr() if cmp_ else 0,
+                       cmp_block_table.data_ptr() if cmp_ else 0,
+                       cmp_sparse_indices.data_ptr() if cmp_ and cmp_sparse_indices is not None else 0,
+                       cu, 0, kv, sinks.data_ptr(), out.data_ptr(), lse.data_ptr(), ws, r.ws_bytes) + r.tail, stream)
+        if rc:
+            _lib.check(rc, "sparse_attn_sharedkv")
+    finally:
+        if staged is not None:
+            ring.release(staged[1], stream)
+    return (out, lse) if return_softmax_lse else out
 
 
 class PreparedBackward:

@@ -13,6 +13,7 @@ bf16/fp16 copy or quantised into the 656-byte fp8 rows of
 from __future__ import annotations
 
 import ctypes as C
+import struct
 from typing import Optional
 
 import torch
@@ -21,6 +22,8 @@ from . import _lib
 
 _DT = {torch.bfloat16: _lib.SAS_DT_BF16, torch.float16: _lib.SAS_DT_FP16}
 FP8_ROW_BYTES = 656
+# the current stream as a hipStream_t value, without a Stream object
+_raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 class PreparedCacheWrite:
@@ -49,9 +52,13 @@ class PreparedCacheWrite:
                    "write_kv_cache")
 
 
-def prepare_kv_cache_write(kv: torch.Tensor, cache: torch.Tensor, block_table: torch.Tensor,
-                           seq_ids: torch.Tensor, positions: torch.Tensor) -> PreparedCacheWrite:
-    """Validate the arguments of :func:`write_kv_cache` and bind them."""
+def _i32(t: torch.Tensor) -> torch.Tensor:
+    return t if t.dtype is torch.int32 and t.is_contiguous() else t.to(torch.int32).contiguous()
+
+
+def _bind(kv, cache, block_table, seq_ids, positions):
+    """Validate and convert: (launch arguments in SasCacheWriteArgs' order,
+    the tensors they point into, device)."""
     if kv.dim() != 2:
         raise ValueError(f"kv must be [N, D], got {tuple(kv.shape)}")
     if kv.dtype not in _DT:
@@ -67,24 +74,44 @@ def prepare_kv_cache_write(kv: torch.Tensor, cache: torch.Tensor, block_table: t
         raise ValueError("cache must hold rows of kv's dtype and width, or uint8 fp8 rows")
     if block_table.dim() != 2:
         raise ValueError("block_table must be [B, max_blocks]")
-    for name, t in (("seq_ids", seq_ids), ("positions", positions)):
-        if t.shape != (N,):
-            raise ValueError(f"{name} must be [N] = [{N}], got {tuple(t.shape)}")
+    if seq_ids.shape != (N,) or positions.shape != (N,):
+        name, t = ("seq_ids", seq_ids) if seq_ids.shape != (N,) else ("positions", positions)
+        raise ValueError(f"{name} must be [N] = [{N}], got {tuple(t.shape)}")
     dev = kv.device
-    if any(t.device != dev for t in (cache, block_table, seq_ids, positions)):
+    if cache.device != dev or block_table.device != dev or seq_ids.device != dev or positions.device != dev:
         raise ValueError("all tensors must be on kv's device")
     if kv.stride(1) != 1 or not cache.is_contiguous():
         raise ValueError("kv rows and cache must be contiguous")
-    bt = block_table.to(torch.int32).contiguous()
-    sid = seq_ids.to(torch.int32).contiguous()
-    pos = positions.to(torch.int32).contiguous()
-    a = _lib.SasCacheWriteArgs(
-        kv=kv.data_ptr(), seq_ids=sid.data_ptr(), positions=pos.data_ptr(),
-        block_table=bt.data_ptr(), cache=cache.data_ptr(),
-        N=N, B=bt.shape[0], D=D, kv_stride=kv.stride(0), bt_stride=bt.shape[1],
-        block_size=cache.shape[1], num_blocks=cache.shape[0],
-        kv_dtype=_DT[kv.dtype], cache_dtype=_lib.SAS_DT_FP8_E4M3_ROW656 if fp8 else _DT[kv.dtype])
-    return PreparedCacheWrite(a, [kv, cache, bt, sid, pos], dev)
+    bt, sid, pos = _i32(block_table), _i32(seq_ids), _i32(positions)
+    nb, bs = cache.shape[0], cache.shape[1]
+    return ((kv.data_ptr(), sid.data_ptr(), pos.data_ptr(), bt.data_ptr(), cache.data_ptr(), N, bt.shape[0], D,
+             kv.stride(0), bt.shape[1], bs, nb, _DT[kv.dtype],
+             _lib.SAS_DT_FP8_E4M3_ROW656 if fp8 else _DT[kv.dtype]), (kv, cache, bt, sid, pos), dev)
+
+
+def prepare_kv_cache_write(kv: torch.Tensor, cache: torch.Tensor, block_table: torch.Tensor,
+                           seq_ids: torch.Tensor, positions: torch.Tensor) -> PreparedCacheWrite:
+    """Validate the arguments of :func:`write_kv_cache` and bind them."""
+    args, keep, dev = _bind(kv, cache, block_table, seq_ids, positions)
+    return PreparedCacheWrite(_lib.SasCacheWriteArgs(*args), list(keep), dev)
+
+
+# SasCacheWriteArgs as packed bytes (five pointers, seven int64, two int32):
+# filling the ctypes structure field by field took a third of a small call
+_ARGS = struct.Struct("@5Q7q2i")
+assert _ARGS.size == C.sizeof(_lib.SasCacheWriteArgs)
+_write_raw = None
+
+
+def _write_bytes():
+    """sas_cache_write_v1 taking its arguments as packed bytes."""
+    global _write_raw
+    if _write_raw is None:
+        f = _lib.lib()["sas_cache_write_v1"]   # a function object of its own: other argument types
+        f.argtypes = [C.c_char_p, C.c_void_p]
+        f.restype = C.c_int
+        _write_raw = f
+    return _write_raw
 
 
 def write_kv_cache(kv: torch.Tensor, cache: torch.Tensor, block_table: torch.Tensor,
@@ -99,4 +126,11 @@ def write_kv_cache(kv: torch.Tensor, cache: torch.Tensor, block_table: torch.Ten
     is negative, or whose block-table entry is -1 or missing, are skipped.
     The rows of one call must go to distinct cache rows.
     """
-    prepare_kv_cache_write(kv, cache, block_table, seq_ids, positions).launch(stream)
+    if stream is not None or not kv.is_cuda:
+        prepare_kv_cache_write(kv, cache, block_table, seq_ids, positions).launch(stream)
+        return
+    # on the current stream, as any conversion made by _bind
+    args, keep, dev = _bind(kv, cache, block_table, seq_ids, positions)
+    rc = _write_bytes()(_ARGS.pack(*args), torch.cuda.current_stream(dev).cuda_stream if _raw is None else _raw(dev.index))
+    if rc:
+        _lib.check(rc, "write_kv_cache")

@@ -875,3 +875,29 @@ def test_dense_runs_match_per_token(name, spec):
     vmax = float(max(inp.ori_kv.abs().max(), inp.cmp_kv.abs().max()))
     assert float((o0 - o1).abs().max()) <= 2 * step * vmax
     assert float((o0 - o1).norm() / o1.norm().clamp_min(1e-9)) < step
+
+
+@pytest.mark.gpu
+def test_signature_cache_takes_new_buffers():
+    """A call of a shape seen before on other buffers, from another stream and
+    with other host lengths, reads its own operands (a resolution holds no
+    address): equal to a freshly prepared call, for host and device lengths."""
+    from dsv4_amd.api import prepare_sparse_attn_sharedkv, sparse_attn_sharedkv
+    side = torch.cuda.Stream()
+    for host in (True, False):
+        for seed in range(3):
+            inp = _small(B=3, H=64, q_lens=[1, 2, 1], kv_lens=[900 + 40 * seed, 700, 333], K=48, seed=seed)
+            if seed == 2:   # the tables' width is part of the signature: keep it
+                inp.seqused_kv[0] = 901
+            d = inp.to("cuda")
+            kw = d.api_kwargs()
+            if not host:
+                kw["cu_seqlens_q"], kw["seqused_kv"] = kw["cu_seqlens_q"].cuda(), kw["seqused_kv"].cuda()
+            ref = prepare_sparse_attn_sharedkv(d.q, **kw)
+            ref.launch()
+            torch.cuda.synchronize()
+            for st in (torch.cuda.current_stream(), side):
+                with torch.cuda.stream(st):
+                    out, lse = sparse_attn_sharedkv(d.q, return_softmax_lse=True, **kw)
+                torch.cuda.synchronize()
+                assert torch.equal(out, ref.out) and torch.equal(lse, ref.lse), (host, seed)
