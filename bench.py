@@ -397,14 +397,16 @@ def bench_backward(dec_inp, pre_inp, atomic_peak=None):
     FLOP per (token, key, head): 2 x (3 x 576 + 2 x 512) = 5504. Row-gradient
     atomics per launch: one fp32 add per (token, key, head group of
     heads_per_workgroup, channel), counted here (with several KV splits the
-    dq shares add atomically too, not counted). The launch's atomic rate
-    against the measured fp32 atomic peak is the bound that applies (the FLOP
-    rate is far below the MFMA peak)."""
+    dq shares add atomically too, not counted); the launch's atomic rate
+    against the measured fp32 atomic peak is the bound that applies there (the
+    FLOP rate is far below the MFMA peak). Prefills sum the rows' gradients
+    key-major: one add per (row of a 64-row tile, channel, 64-token segment,
+    32-head group), and their matrix work bounds them."""
     from dsv4_amd import cases
     from dsv4_amd.api import prepare_sparse_attn_sharedkv_backward, sparse_attn_sharedkv
     res = {"kernel": "sas_bwd64_kernel (64-head workgroups, q in registers; MFMA scores, dq and dkv; "
-                     "fp32 atomics for dkv); sas_bwd_kernel for H not a multiple of 64; prefills: the "
-                     "window rows' dkv by sas_bwd_win_kernel beside it on a side stream",
+                     "fp32 atomics for dkv); sas_bwd_kernel for H not a multiple of 64; prefills: "
+                     "sas_bwd_dq_kernel (dq, token-major) and sas_bwd_keys_kernel (row gradients, key-major)",
            "flop_per_pair_head": BWD_FLOP_PER_PAIR_HEAD}
     for key, inp, steps in (("decode", dec_inp, 50), ("prefill", pre_inp, 3)):
         if inp is None:
@@ -421,18 +423,19 @@ def bench_backward(dec_inp, pre_inp, atomic_peak=None):
         tfl = flop / (us * 1e-6) / 1e12
         hpw = 64 if inp.cfg.H % 64 == 0 else 32 if inp.cfg.H % 32 == 0 else 16
         D = inp.q.shape[-1]
-        # the library's default: the key-major window pass for prefills (at
-        # least 64 query tokens per batch), whose window rows take one add
-        # per (row, 16-head group, channel) instead of one per (token, row)
+        # the library's default: the prefill path from 64 query tokens per
+        # batch on (top-k lists dense below the causal threshold, as here)
         win_pass = inp.q.shape[0] >= 64 * len(inp.q_lens)
-        win_pairs, win_rows = 0, 0
-        for aq, akv in zip(inp.q_lens, inp.kv_lens):
-            wl = inp.cfg.win_left
-            win_pairs += sum(min(akv - aq + s, wl) + 1 for s in range(aq) if akv - aq + s >= 0)
-            win_rows += akv - max(akv - aq - wl, 0) if aq > 0 else 0
         atomics = pairs * (inp.cfg.H // hpw) * D
         if win_pass:
-            atomics = ((pairs - win_pairs) * (inp.cfg.H // hpw) + win_rows * (inp.cfg.H // 16)) * D
+            tiles = 0
+            for aq, akv in zip(inp.q_lens, inp.kv_lens):
+                for s0 in range(0, aq, 64):
+                    lo, hi = akv - aq + s0, akv - aq + min(s0 + 64, aq) - 1   # causal positions of the segment
+                    tiles += hi // 64 - max(0, lo - inp.cfg.win_left) // 64 + 1
+                    if inp.cfg.scenario > 1:
+                        tiles += -(-((hi + 1) // inp.cfg.cmp_ratio) // 64)
+            atomics = tiles * 64 * D * (inp.cfg.H // 32)
         rate = atomics / (us * 1e-6) / 1e9
         res[key] = dict(workload=inp.cfg.name, us_per_call=round(us, 1), useful_flop=flop,
                         tflops=round(tfl, 2), mfma_frac=round(tfl / BF16_PEAK_TFLOPS, 5),
@@ -441,7 +444,7 @@ def bench_backward(dec_inp, pre_inp, atomic_peak=None):
                         atomic_frac=round(rate / atomic_peak, 3) if atomic_peak else None,
                         atomic_frac_of="peaks.fp32_atomic_measured_g_per_s")
         if win_pass:
-            # the same launch with per-token adds for the window rows too
+            # the same launch with per-token adds for every row
             del pb
             pb = prepare_sparse_attn_sharedkv_backward(dout, inp.q, out, lse, window_pass=False, **kw)
             ms, _ = time_launches(lambda i, st: pb.launch(st), 1, steps, 1)

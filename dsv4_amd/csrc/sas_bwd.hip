@@ -568,7 +568,8 @@ __global__ void __launch_bounds__(512) sas_bwd64_kernel(const BwdParams bp) {
 // differs from theirs only in fp32 summation order. Row validity follows
 // resolve(): position below act_kv, block inside the table, table entry
 // inside the cache. It runs beside the per-token kernel on a side stream
-// (SideStream below); sas_bwd_v1 chooses it for prefills.
+// (SideStream below); sas_bwd_v1 chooses it for prefills that do not take the
+// prefill path (sas_bwd_pre.hip: no workspace given, or H not a multiple of 32).
 constexpr int kWinRows = 64;   // positions per tile (16 per wave)
 
 template <int D, typename QT>
@@ -874,7 +875,7 @@ int launch_tokens(const BwdParams& bp, const SasFwdArgs* a, bool b64, int ng, in
 // Query tokens share rows from about 64 tokens per batch on (as for the
 // window pass), and its head groups are 32 wide.
 #ifndef SAS_BWD_DENSE
-#define SAS_BWD_DENSE 8
+#define SAS_BWD_DENSE 7
 #endif
 struct PrePlan {
   bool on, sparse;   // sparse: some tokens may need per-token adds for their compressed rows
@@ -889,9 +890,12 @@ PrePlan plan_prefill(const SasFwdArgs* a) {
          ((a->flags & SAS_BWD_WINDOW_KEYS) || a->T >= 64 * a->B);
   if (!r.on) return r;
   // A token with n compressed rows below its causal threshold and a list of K
-  // of them costs the key-major pass n row products (~0.2 ns each with 64
-  // heads when the chip is full) and the per-token kernel min(n, K) atomic
-  // adds per channel (1.77 ns): key-major up to n = 8 K.
+  // of them costs the key-major pass n row products and the per-token kernel
+  // min(n, K) atomic adds per channel (and its own slower products). 1024
+  // tokens, 64 heads, all tokens key-major against all per token: K = 64, n
+  // about 512 / 1024 / 1536 rows, 417 against 479, 559 / 461, 676 / 469 us; K =
+  // 256, n about 512 / 1024 / 2048 / 3072, 437 against 702, 584 / 799, 879 /
+  // 810, 1148 / 803 us. They meet between 7 K and 11 K.
   const long long cap = a->scenario >= SAS_CFA ? a->cmp_bt_stride * a->cmp_block_size : 0;
   const long long dense = a->scenario == SAS_SCFA ? std::min<long long>(INT_MAX, SAS_BWD_DENSE * a->K) : INT_MAX;
   r.dense_thr = (int)dense;

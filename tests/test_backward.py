@@ -513,7 +513,7 @@ def test_gpu_backward_h48_d512_matches_oracle():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,spec", [
-    # tokens on both sides of the density rule (8 K rows): dense ones by the
+    # tokens on both sides of the density rule (a few K rows): dense ones by the
     # key-major pass, the others by per-token adds; 64- and 32-head groups
     ("both_h64", dict(B=1, H=64, q_lens=[400], kv_lens=[400], K=8)),
     ("both_h32", dict(B=2, H=32, q_lens=[270, 90], kv_lens=[330, 500], K=8, D=512, bs=16)),
