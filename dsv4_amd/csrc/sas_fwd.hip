@@ -2083,15 +2083,17 @@ bool win_runs(const SasFwdArgs* a, const Plan& pl) {
          a->head_waves == 0 && (long long)a->T * pl.nhg > sas::device_cus();
 }
 
-// Dense compressed calls walk runs of tokens too, from four rounds of
-// 64-head workgroups on and where batches are long enough to have runs (64
-// heads, ratio 128: D = 576, 512 tokens 32.6 against 28.0 us, 1000 tokens 50.6
-// against 52.0, 2000 tokens 90 against 97; D = 512 with 128 heads, 512 tokens
-// 42 against 53; 300 batches of 3 tokens 69 against 61).
+// Dense compressed calls walk runs of tokens too, from four (D = 512) or eight
+// (D = 576, whose two workgroups per CU spill a little) rounds of 64-head
+// workgroups on and where batches are long enough to have runs (64 heads,
+// ratio 128: D = 576, 512 tokens 32.6 against 28.0 us, 1000 tokens 50.6 against
+// 52.0, 2000 tokens 90 against 97, 3 x 301 tokens with 128 heads and a 64-row
+// window 86.8 against 86.1; D = 512 with 128 heads, 512 tokens 42 against 53;
+// 300 batches of 3 tokens 69 against 61).
 bool dense_runs(const SasFwdArgs* a, const Plan& pl) {
   return a->scenario == SAS_CFA && a->kv_dtype == a->q_dtype && a->H % 64 == 0 && a->win_left + kRunTokens <= kDenseWinRows &&
          a->K <= kDenseCmpRows && pl.nsplit == 1 && a->head_waves == 0 && a->waves == 0 && a->T >= 64 * a->B &&
-         a->T * (a->H / 64) >= 4LL * sas::device_cus();
+         a->T * (a->H / 64) >= (a->D == 512 ? 4LL : 8LL) * sas::device_cus();
 }
 
 template <int HW, int NW, int D, typename QT, int KVF, bool EXW = false>

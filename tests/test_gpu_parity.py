@@ -840,13 +840,13 @@ def test_window_runs_bsnd_padding():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,spec", [
-    ("h64", dict(B=1, H=64, q_lens=[1100], kv_lens=[1100], ratio=16)),
+    ("h64", dict(B=1, H=64, q_lens=[2050], kv_lens=[2050], ratio=16)),
     ("h128_d512_fp16", dict(B=2, H=128, q_lens=[400, 130], kv_lens=[3400, 130], ratio=32, D=512, bs=16, dtype=torch.float16)),
     # the limits of the run's tables (128 window rows + runs, 128 compressed), a compressed row per token
     ("limits", dict(B=1, H=64, q_lens=[1030], kv_lens=[1031], ratio=8, D=512, win=128)),
-    ("ratio1_win1", dict(B=9, H=64, q_lens=[128] * 9, kv_lens=[128] * 9, ratio=1, win=0)),
-    ("short_kv", dict(B=2, H=64, q_lens=[800, 300], kv_lens=[350, 3], ratio=4, win=40)),
-    ("missing_blocks", dict(B=1, H=64, q_lens=[1050], kv_lens=[1050], ratio=16, bs=16)),
+    ("ratio1_win1", dict(B=17, H=64, q_lens=[128] * 17, kv_lens=[128] * 17, ratio=1, win=0)),
+    ("short_kv", dict(B=2, H=64, q_lens=[800, 300], kv_lens=[350, 3], ratio=4, win=40, D=512)),
+    ("missing_blocks", dict(B=1, H=128, q_lens=[1050], kv_lens=[1050], ratio=16, bs=16)),
 ])
 def test_dense_runs_match_per_token(name, spec):
     """Dense compressed prefills by runs of tokens against the one-workgroup-
