@@ -182,7 +182,8 @@ int sas_fwd_plan(const SasFwdArgs* a, int32_t* num_splits, size_t* workspace_byt
 
 /*
  * Launch the fused forward on `stream`: one workgroup per (token, head group,
- * KV split), gather through block tables into LDS, bf16/fp16 MFMA for QK^T and
+ * KV split), or per run of tokens (window-only and dense compressed prefills),
+ * gather through block tables into LDS, bf16/fp16 MFMA for QK^T and
  * PV, sink-seeded online softmax, and (when splits > 1) the LSE combine.
  * Replaces the jitted callable of kernel.py:156-178 / api.py:372-384.
  */
