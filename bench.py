@@ -400,7 +400,7 @@ def bench_backward(dec_inp, pre_inp, atomic_peak=None):
     dq shares add atomically too, not counted); the launch's atomic rate
     against the measured fp32 atomic peak is the bound that applies there (the
     FLOP rate is far below the MFMA peak). Prefills sum the rows' gradients
-    key-major: one add per (row of a 64-row tile, channel, 64-token segment,
+    key-major: one add per (row of a 64-row tile, channel, 96-token segment,
     32-head group), and their matrix work bounds them."""
     from dsv4_amd import cases
     from dsv4_amd.api import prepare_sparse_attn_sharedkv_backward, sparse_attn_sharedkv
@@ -430,8 +430,8 @@ def bench_backward(dec_inp, pre_inp, atomic_peak=None):
         if win_pass:
             tiles = 0
             for aq, akv in zip(inp.q_lens, inp.kv_lens):
-                for s0 in range(0, aq, 64):
-                    lo, hi = akv - aq + s0, akv - aq + min(s0 + 64, aq) - 1   # causal positions of the segment
+                for s0 in range(0, aq, 96):
+                    lo, hi = akv - aq + s0, akv - aq + min(s0 + 96, aq) - 1   # causal positions of the segment
                     tiles += hi // 64 - max(0, lo - inp.cfg.win_left) // 64 + 1
                     if inp.cfg.scenario > 1:
                         tiles += -(-((hi + 1) // inp.cfg.cmp_ratio) // 64)

@@ -26,6 +26,7 @@ struct BwdParams {
   int dense_thr;        // tokens with a causal threshold up to this have their compressed rows' gradients
                         // summed by the key-major pass; the others add per token
   int sparse_only;      // per-token kernels: 1 takes only the tokens beyond dense_thr
+  int key_seg;          // key-major pass: tokens per segment
   int seg_groups;       // key-major pass: (batch, segment) slots of the grid
   int cmp_tiles;        // key-major pass: compressed row tiles per segment
   int win_tiles_seg;    // key-major pass: window row tiles per segment
@@ -81,7 +82,6 @@ __device__ __forceinline__ float sum16(float x) {
 int launch_bwd_prefill(const BwdParams& bp, int D, int q_dtype, hipStream_t st);
 // heads per workgroup of sas_bwd_dq_kernel
 inline int bwd_dq_heads(int H) { return H % 64 == 0 ? 64 : 32; }
-constexpr int kKeySeg = 64;    // tokens per segment of the key-major pass
 constexpr int kKeyRows = 64;   // rows per tile of the key-major pass
 
 }  // namespace sas

@@ -879,7 +879,7 @@ int launch_tokens(const BwdParams& bp, const SasFwdArgs* a, bool b64, int ng, in
 #endif
 struct PrePlan {
   bool on, sparse;   // sparse: some tokens may need per-token adds for their compressed rows
-  int dense_thr;
+  int dense_thr, key_seg;
   long long seg_groups, cmp_tiles, win_tiles;
   size_t ws;
 };
@@ -901,9 +901,22 @@ PrePlan plan_prefill(const SasFwdArgs* a) {
   r.dense_thr = (int)dense;
   r.sparse = a->scenario == SAS_SCFA && cap > dense;
   const long long rows = a->scenario == SAS_CFA ? std::min<long long>(cap, a->K) : std::min(cap, dense);
-  r.seg_groups = a->T / kKeySeg + a->B;
   r.cmp_tiles = (rows + kKeyRows - 1) / kKeyRows;
-  r.win_tiles = std::min<long long>(((long long)a->win_left + kKeySeg + 2 * (kKeyRows - 1)) / kKeyRows,
+  // Segments: the longest that still give the key-major pass about three
+  // rounds of workgroups (window tiles, and half of the compressed ones, on
+  // average). Longer ones spread a workgroup's rows and adds over more tokens,
+  // shorter ones fill the CUs (backward, 64 heads, segments of 32 / 64 / 96
+  // tokens: 512 tokens 150 / 211 / 274 us, 2048 tokens 765 / 789 / 776, 6000
+  // tokens 3113 / 3034 / 2922; 2726 packed tokens with 128 heads 1427 / 1417 /
+  // 1278; 16 tokens: 171 and 1596). Near the line it can miss: three
+  // sequences of 500 to 2000 tokens take 96 and 1240 us, with 64 1152.
+  for (int seg : {96, 64, 32}) {
+    r.key_seg = seg;
+    const double wgs = (double)a->T / seg * (a->H / 32) * (((double)a->win_left + seg) / kKeyRows + 1 + r.cmp_tiles / 2.0);
+    if (wgs >= 2.75 * device_cus()) break;
+  }
+  r.seg_groups = a->T / r.key_seg + a->B;
+  r.win_tiles = std::min<long long>(((long long)a->win_left + r.key_seg + 2 * (kKeyRows - 1)) / kKeyRows,
                                     (a->ori_bt_stride * a->ori_block_size + kKeyRows - 1) / kKeyRows);
   r.ws = (size_t)a->T * a->H * sizeof(float);
   if ((r.sparse && nslots > kMaxSlots) || r.ws == 0 ||
@@ -1043,6 +1056,7 @@ extern "C" int sas_bwd_v1(const SasBwdArgs* ba, void* stream) {
     bp.dq_direct = direct;
     bp.dense_thr = pre.dense_thr;
     bp.npass = (int)((nslots + kMaxSlots - 1) / kMaxSlots);
+    bp.key_seg = pre.key_seg;
     bp.seg_groups = (int)pre.seg_groups;
     bp.cmp_tiles = (int)pre.cmp_tiles;
     bp.win_tiles_seg = (int)pre.win_tiles;

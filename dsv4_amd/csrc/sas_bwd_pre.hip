@@ -21,7 +21,7 @@
 // Forward + backward of a 4096-token, 64-head, top-k 512 step: 4.35 ms with
 // per-token adds (the window rows key-major beside them), 2.12 ms here (dq
 // 0.78, rows 1.11 ms); the backward of 2726 packed tokens with 128 heads 2.61
-// against 1.41 ms.
+// against 1.20 ms.
 
 #include "sas_bwd.h"
 
@@ -269,7 +269,7 @@ __global__ void __launch_bounds__(128 * NG) sas_bwd_dq_kernel(const BwdParams bp
 // row gradients, key-major
 // ---------------------------------------------------------------------------
 //
-// Workgroup = (segment of kKeySeg consecutive tokens of one batch, 32-head
+// Workgroup = (segment of key_seg consecutive tokens of one batch, 32-head
 // group, tile of 64 window or compressed rows), 8 waves. Its unit is one token
 // (32 heads): q and dO reach LDS by DMA (two buffers, 139 KB), then
 //   S[head][row] = Q . K^T and dP = dO . V^T   (16x16x32 MFMA; wave w: rows
@@ -324,7 +324,7 @@ __global__ void __launch_bounds__(512) sas_bwd_keys_kernel(const BwdParams bp) {
         kvi = p.act_kv[i];
         ae = qpi < 0 ? 0 : max(0, min(aqi, min(nxt, p.T) - qpi));
       }
-      const int n = (ae + kKeySeg - 1) / kKeySeg;
+      const int n = (ae + bp.key_seg - 1) / bp.key_seg;
       int s = n;
 #pragma unroll
       for (int d = 1; d < 64; d <<= 1) { const int v = __shfl_up(s, d); s += lane >= d ? v : 0; }
@@ -347,7 +347,7 @@ __global__ void __launch_bounds__(512) sas_bwd_keys_kernel(const BwdParams bp) {
   akv = __builtin_amdgcn_readfirstlane(akv);
   const int sg0 = akv - aq;                     // causal position of the batch's first token
   // token offsets [a0, a1) of the segment in the batch
-  int a0 = seg * kKeySeg, a1 = min(a0 + kKeySeg, aqe);
+  int a0 = seg * bp.key_seg, a1 = min(a0 + bp.key_seg, aqe);
   if (a0 + sg0 < 0) a0 = min(a1, -sg0);         // tokens before position 0 attend no row
   const bool cmp = tile < bp.cmp_tiles;
   int p0;                                       // the tile's first position

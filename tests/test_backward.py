@@ -524,7 +524,8 @@ def test_gpu_backward_h48_d512_matches_oracle():
     # more key slots than one resolution pass holds, and lists past 2048 entries
     ("dense_passes", dict(B=1, H=64, q_lens=[70], kv_lens=[5200], K=0, scenario=2)),
     ("long_lists", dict(B=1, H=128, q_lens=[66], kv_lens=[8600], K=2100, D=512, win=1)),
-    # segment and tile edges: 63, 64, 65 and 129 tokens, windows off the tile grid
+    # segment and tile edges, windows off the tile grid; 96-token segments
+    ("long_segments", dict(B=2, H=128, q_lens=[1100, 97], kv_lens=[1100, 500], K=24, win=90, D=512, dtype=torch.float16)),
     ("edges", dict(B=4, H=32, q_lens=[63, 64, 65, 129], kv_lens=[63, 191, 65, 400], K=40, win=66, bs=16)),
 ])
 def test_gpu_backward_prefill_path(name, spec):
