@@ -898,8 +898,11 @@ PrePlan plan_prefill(const SasFwdArgs* a) {
   // 810, 1148 / 803 us. They meet between 7 K and 11 K.
   const long long cap = a->scenario >= SAS_CFA ? a->cmp_bt_stride * a->cmp_block_size : 0;
   const long long dense = a->scenario == SAS_SCFA ? std::min<long long>(INT_MAX, SAS_BWD_DENSE * a->K) : INT_MAX;
-  r.dense_thr = (int)dense;
+  // Thresholds follow the sequences, not the table: where a table has at most
+  // `dense` rows, every token is key-major, also one whose threshold lies past
+  // the table's end (no per-token launch would take it).
   r.sparse = a->scenario == SAS_SCFA && cap > dense;
+  r.dense_thr = r.sparse ? (int)dense : INT_MAX;
   const long long rows = a->scenario == SAS_CFA ? std::min<long long>(cap, a->K) : std::min(cap, dense);
   r.cmp_tiles = (rows + kKeyRows - 1) / kKeyRows;
   // Segments: the longest that still give the key-major pass about three

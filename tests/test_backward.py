@@ -549,3 +549,48 @@ def test_gpu_backward_prefill_path(name, spec):
     _check_against_oracle(name, inp, *got, r)
     _check_against_oracle(f"{name} prepared", inp, *pb.result(), r)
     assert torch.equal(pb.dq.to(got[0].dtype).cpu(), got[0].cpu())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,D,bs", [(64, 576, 64), (32, 512, 16)])
+def test_gpu_backward_table_narrower_than_the_sequences(H, D, bs):
+    """A compressed block table that ends before the causal thresholds: the
+    entries past it are not attended, and every token's gradients are still
+    written (a few times K rows lie between the table's end and the largest
+    threshold, on both sides of the density rule)."""
+    from dataclasses import replace
+    from dsv4_amd.api import (prepare_sparse_attn_sharedkv_backward, sparse_attn_sharedkv,
+                              sparse_attn_sharedkv_backward)
+    from tests.test_gpu_parity import _small
+    K, cap = 32, 64
+    inp = _small(B=2, H=H, q_lens=[80, 70], kv_lens=[4000, 330], K=K, D=D, bs=bs)
+    g = torch.Generator().manual_seed(43)
+    idx = torch.full_like(inp.cmp_idx, -1)
+    inside = torch.full_like(inp.cmp_idx, -1)
+    for t in range(idx.shape[0]):
+        thr = (4000 - 80 + t + 1) // 4 if t < 80 else (330 - 70 + t - 80 + 1) // 4
+        n = min(K // 2, thr)
+        head = torch.randperm(min(cap, thr), generator=g)[:n].to(torch.int32)
+        inside[t, 0, :n] = head
+        idx[t, 0, :n] = head
+        if thr > cap:
+            idx[t, 0, n:] = cap + torch.randperm(thr - cap, generator=g)[:K - n].to(torch.int32) \
+                if thr - cap >= K - n else -1
+    inp = replace(inp, cmp_idx=idx, cmp_bt=inp.cmp_bt[:, :cap // bs].contiguous())
+    d = inp.to("cuda")
+    kw = d.api_kwargs()
+    out, lse = sparse_attn_sharedkv(d.q, return_softmax_lse=True, **kw)
+    dout = torch.randn(out.shape, generator=g).to(inp.q.dtype)
+    r = _oracle_bwd(replace(inp, cmp_idx=inside), dout, out, lse)
+    dout = dout.cuda()
+    # fill the blocks that the call's own tensors are likely to get (one of
+    # them may be left unwritten)
+    torch.full(d.q.shape, float("nan"), dtype=d.q.dtype, device="cuda")
+    torch.full(lse.shape, float("nan"), device="cuda")
+    got = sparse_attn_sharedkv_backward(dout, d.q, out, lse, **kw)
+    pb = prepare_sparse_attn_sharedkv_backward(dout, d.q, out, lse, **kw)
+    pb.launch()
+    torch.cuda.synchronize()
+    assert all(torch.isfinite(x).all() for x in (*got, *pb.result()))
+    _check_against_oracle(f"narrow table H{H}", inp, *got, r)
+    _check_against_oracle(f"narrow table H{H} prepared", inp, *pb.result(), r)
