@@ -21,6 +21,7 @@ struct BwdParams {
   int win_tiles;        // sas_bwd_win_kernel: 64-position row tiles per batch
   // key-major path (sas_bwd_pre.hip)
   float* delta;         // [T, H] fp32 workspace: Delta = dO . O
+  uint8_t* nonfinite;   // [T, H / 16, 2] workspace: 1 if the heads' q (in that half of the channels) or dO has a NaN or Inf
   int npass;            // sas_bwd_dq_kernel: slot ranges of slots_per_split a workgroup walks
   int dq_direct;        // 1: dq is in the query dtype and written whole
   int dense_thr;        // tokens with a causal threshold up to this have their compressed rows' gradients

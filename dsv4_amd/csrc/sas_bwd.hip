@@ -921,7 +921,7 @@ PrePlan plan_prefill(const SasFwdArgs* a) {
   r.seg_groups = a->T / r.key_seg + a->B;
   r.win_tiles = std::min<long long>(((long long)a->win_left + r.key_seg + 2 * (kKeyRows - 1)) / kKeyRows,
                                     (a->ori_bt_stride * a->ori_block_size + kKeyRows - 1) / kKeyRows);
-  r.ws = (size_t)a->T * a->H * sizeof(float);
+  r.ws = (size_t)a->T * a->H * sizeof(float) + (size_t)a->T * (a->H / 8);   // Delta, non-finite marks
   if ((r.sparse && nslots > kMaxSlots) || r.ws == 0 ||
       (double)(r.cmp_tiles + r.win_tiles) * (r.seg_groups + 64) * (a->H / 32) > 2e9)
     return PrePlan{};
@@ -1056,6 +1056,7 @@ extern "C" int sas_bwd_v1(const SasBwdArgs* ba, void* stream) {
   }
   if (pre.on && have_ws && (direct || !capturing || (a->flags & SAS_BWD_WINDOW_KEYS))) {
     bp.delta = (float*)a->workspace;
+    bp.nonfinite = (uint8_t*)(bp.delta + (size_t)a->T * a->H);
     bp.dq_direct = direct;
     bp.dense_thr = pre.dense_thr;
     bp.npass = (int)((nslots + kMaxSlots - 1) / kMaxSlots);

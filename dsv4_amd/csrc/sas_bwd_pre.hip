@@ -93,6 +93,16 @@ __global__ void __launch_bounds__(128 * NG) sas_bwd_dq_kernel(const BwdParams bp
   }
   const float lse2 = p.lse[th] * kLog2e;
   float dl = 0.f;
+  // the token's non-finite marks: q (0 times it) or dO (Delta). Stored last: the
+  // chunk loop's first wait would include it
+  auto mark = [&] {
+    float z[2] = {dl, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KSH; ++ks)
+      z[ks & 1] = dot2<QT>(qf[ks].w, 0, dot2<QT>(qf[ks].z, 0, dot2<QT>(qf[ks].y, 0, dot2<QT>(qf[ks].x, 0, z[ks & 1]))));
+    const bool nf = __ballot(!(fabsf(z[0] + z[1]) < INFINITY)) != 0;
+    if (lane == 0) bp.nonfinite[(size_t)t * (p.H / 8) + (k.hg * NG + g) * 2 + hh] = nf;
+  };
 
   f32x4 acc[DQT];
 #pragma unroll
@@ -124,7 +134,10 @@ __global__ void __launch_bounds__(128 * NG) sas_bwd_dq_kernel(const BwdParams bp
     resolve<256, D * 2>(p, k, tid, lane, wave, [] {});
     if (pass == 0) {
       dl = lds_dl[16 * g + c16];   // behind resolve()'s barriers
-      if (k.thr > bp.dense_thr) return;   // the per-token kernel's token
+      if (k.thr > bp.dense_thr) {         // the per-token kernel's token
+        mark();
+        return;
+      }
       if (hh == 0 && g4 == 0) bp.delta[th] = k.padded ? 0.f : dl;
     }
     const int nvalid = __builtin_amdgcn_readfirstlane(k.nvalid);
@@ -263,6 +276,7 @@ __global__ void __launch_bounds__(128 * NG) sas_bwd_dq_kernel(const BwdParams bp
 #pragma unroll
     for (int j = 0; j < DQT; ++j) *reinterpret_cast<f32x4*>(dst + j * 16) = acc[j];
   }
+  mark();
 }
 
 // ---------------------------------------------------------------------------
@@ -282,6 +296,21 @@ __global__ void __launch_bounds__(128 * NG) sas_bwd_dq_kernel(const BwdParams bp
 // Every q / dO element is read from LDS by four waves for S and by one for
 // dkv. All tiles of a (segment, head group) run on one XCD next to each
 // other, so the tokens' q / dO stream through its L2 once.
+//
+// A unit's products run over every row of the tile, those the token does not
+// attend with P = dS = 0. A NaN or Inf in q or dO would reach them as 0 x Inf:
+// in a segment that holds one (by sas_bwd_dq_kernel's marks) such elements are
+// cleared in LDS before the dkv products, and the rows the token does attend
+// get their NaN through P and dS alone. The marks take 0.5 % of the 4096-token
+// step (looked for unit by unit instead, in S and dP: 1.5 %).
+template <typename QT>
+__device__ __forceinline__ uint32_t finite2(uint32_t w) {   // two packed values, non-finite ones as 0
+  constexpr uint32_t E = std::is_same<QT, __bf16>::value ? 0x7f80u : 0x7c00u;   // exponent all ones
+  if ((w & E) == E) w &= 0xffff0000u;
+  if ((w >> 16 & E) == E) w &= 0xffffu;
+  return w;
+}
+
 template <int D, typename QT>
 __global__ void __launch_bounds__(512) sas_bwd_keys_kernel(const BwdParams bp) {
   constexpr int CH = D / 8, OCH = kDV / 8;     // 16-byte chunks per q / dO row
@@ -381,7 +410,9 @@ __global__ void __launch_bounds__(512) sas_bwd_keys_kernel(const BwdParams bp) {
     lds_c[0][tid] = 0;
     lds_c[1][tid] = 0;
   }
-  __syncthreads();
+  // (a segment has fewer tokens than the workgroup threads)
+  const bool nf = __syncthreads_or(
+      tid < a1 - a0 && reinterpret_cast<const uint32_t*>(bp.nonfinite)[((size_t)qp + a0 + tid) * nhg + hg] != 0);
   const int rt = wave & 3, ht = wave >> 2;
   uint4 kf[KS];
   const uint64_t ra = lds_r[16 * rt + c16];
@@ -557,6 +588,18 @@ __global__ void __launch_bounds__(512) sas_bwd_keys_kernel(const BwdParams bp) {
     }
     lds_barrier();
     if (list && tid < kKeyRows) lds_c[buf][tid] = 0;
+    if (nf) {
+      auto clear = [&](uint4* b, int n) {
+#pragma unroll 1
+        for (int i = tid; i < n; i += 512) {
+          const uint4 v = b[i];
+          b[i] = make_uint4(finite2<QT>(v.x), finite2<QT>(v.y), finite2<QT>(v.z), finite2<QT>(v.w));
+        }
+      };
+      clear(lds_q[buf], 32 * CH);
+      clear(lds_o[buf], 32 * OCH);
+      lds_barrier();
+    }
     {
       uint4 ads[4], ap[4];
 #pragma unroll

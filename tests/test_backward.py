@@ -594,3 +594,63 @@ def test_gpu_backward_table_narrower_than_the_sequences(H, D, bs):
     assert all(torch.isfinite(x).all() for x in (*got, *pb.result()))
     _check_against_oracle(f"narrow table H{H}", inp, *got, r)
     _check_against_oracle(f"narrow table H{H} prepared", inp, *pb.result(), r)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", ["q_nan", "q_inf_rope", "dout_inf", "dout_nan"])
+@pytest.mark.parametrize("spec", [
+    dict(H=64, q_lens=[200], kv_lens=[400], K=24),
+    dict(H=32, q_lens=[130], kv_lens=[700], K=8, bs=16, dtype=torch.float16),
+    dict(H=32, q_lens=[150], kv_lens=[300], K=0, scenario=2, win=40),
+], ids=["topk", "both_passes", "dense"])
+def test_gpu_backward_non_finite_token_stays_in_its_rows(spec, what):
+    """A token with a NaN or Inf in one head's q or dout makes the gradients of
+    the rows it attends non-finite, and no others: they, every other token's
+    dq and every other head's sink gradient are those of the call without it."""
+    from dsv4_amd.api import sparse_attn_sharedkv, sparse_attn_sharedkv_backward
+    from tests.test_gpu_parity import _small
+    inp = _small(B=1, **spec)
+    d = inp.to("cuda")
+    kw = d.api_kwargs()
+    g = torch.Generator().manual_seed(47)
+    D, T, H = inp.q.shape[-1], inp.q.shape[0], spec["H"]
+    dout = torch.randn((T, H, 512), generator=g).to(inp.q.dtype).cuda()
+    t, h = 77, 5
+    clean_out, clean_lse = sparse_attn_sharedkv(d.q, return_softmax_lse=True, **kw)
+    q, bad_dout = d.q.clone(), dout.clone()
+    if what == "q_nan":
+        q[t, h, 100] = float("nan")
+    elif what == "q_inf_rope":
+        q[t, h, D - 3] = float("inf")
+    else:
+        bad_dout[t, h, 300] = float("inf" if what == "dout_inf" else "nan")
+    out, lse = sparse_attn_sharedkv(q, return_softmax_lse=True, **kw)
+    got = sparse_attn_sharedkv_backward(bad_dout, q, out, lse, **kw)
+    # the call without the token's contributions
+    dout[t] = 0
+    ref = sparse_attn_sharedkv_backward(dout, d.q, clean_out, clean_lse, **kw)
+    torch.cuda.synchronize()
+    others = [i for i in range(T) if i != t]
+    assert torch.equal(got[0][others], ref[0][others])
+    heads = [i for i in range(H) if i != h]
+    sg = spec["kv_lens"][0] - T + t
+    win = spec.get("win", 127)
+
+    def rows(table, positions, bs):
+        return torch.tensor([int(table[0, p // bs]) * bs + p % bs for p in positions])
+
+    sets = [(got[1], ref[1], rows(inp.ori_bt, range(max(0, sg - win), sg + 1), inp.ori_kv.shape[1]))]
+    if got[2] is not None:
+        thr = (sg + 1) // 4
+        pos = [int(x) for x in inp.cmp_idx[t, 0] if 0 <= int(x) < thr] if spec["K"] else range(thr)
+        sets.append((got[2], ref[2], rows(inp.cmp_bt, pos, inp.cmp_kv.shape[1])))
+    for name, (a, b, hit) in zip(("ori", "cmp"), sets):
+        a, b = a.cpu().reshape(-1, D), b.cpu().reshape(-1, D)
+        assert not torch.isfinite(a[hit]).all(dim=1).any(), f"{name}: an attended row stayed finite"
+        free = torch.ones(a.shape[0], dtype=torch.bool)
+        free[hit] = False
+        assert torch.isfinite(a[free]).all(), f"{name}: {int((~torch.isfinite(a[free])).any(1).sum())} other rows hit"
+        # fp32 sums over the tokens in another order
+        assert float((a[free] - b[free]).abs().max()) <= 1e-5 * float(b[free].abs().max()), name
+    snk = got[3][heads]
+    assert torch.isfinite(snk).all()
