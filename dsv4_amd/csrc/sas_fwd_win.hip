@@ -312,6 +312,8 @@ __global__ void __launch_bounds__(256) sas_fwd_win_kernel(const FwdParams p, con
 // registers a wave each): one, with four slots and a deeper DMA lead, took
 // 520 us for 8192 tokens, 64 heads, D = 512, ratio 128; two take 360, the
 // one-workgroup-per-token kernel 452.
+__device__ const uint4 kZeroRow[576 * 2 / 16] = {};   // a missing row's bytes: finite, whatever the caller's hold
+
 template <int D, typename QT>
 __global__ void __launch_bounds__(256, 2) sas_fwd_dense_kernel(const FwdParams p, const int run) {
   // slot: the 32 rows' latent chunks [32][64] (chunk c of row r at c ^
@@ -363,7 +365,7 @@ __global__ void __launch_bounds__(256, 2) sas_fwd_dense_kernel(const FwdParams p
     r.steps = (r.n + 31) >> 5;
     return r;
   };
-  const uint64_t spare = reinterpret_cast<uint64_t>(p.q) + (size_t)rn.r0 * p.H * D * 2;   // a row of finite values
+  const uint64_t spare = reinterpret_cast<uint64_t>(kZeroRow);
   auto row_addr = [&](const Rows& r, int j) {
     j = max(min(j, r.n - 1), 0);
     return tab[j < r.nwin ? r.wb + j : kDenseWinRows + j - r.nwin];
@@ -379,7 +381,7 @@ __global__ void __launch_bounds__(256, 2) sas_fwd_dense_kernel(const FwdParams p
       ps = 0;
       pr = rows_of(pt < rn.r1 ? pt : rn.r1 - 1);
     }
-    // (past the run, and for a missing row: finite bytes, masked out)
+    // (past the run, and for a missing row: zero bytes, masked out)
     pl = row_addr(pr, ps * 32 + 8 * wave + (lane & 7));
     if (ROPE) pp = row_addr(pr, ps * 32 + 8 * wave + (lane >> 3));
     if (pt >= rn.r1) pl = pp = 0;

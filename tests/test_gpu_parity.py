@@ -901,3 +901,29 @@ def test_signature_cache_takes_new_buffers():
                     out, lse = sparse_attn_sharedkv(d.q, return_softmax_lse=True, **kw)
                 torch.cuda.synchronize()
                 assert torch.equal(out, ref.out) and torch.equal(lse, ref.lse), (host, seed)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,T", [(512, 1040), (576, 2060)])
+def test_dense_runs_missing_rows_beside_a_non_finite_query(D, T):
+    """A token with a non-finite query, the first of a run, leaves the other
+    tokens of its run alone, missing cache rows or not."""
+    from dsv4_amd.api import prepare_sparse_attn_sharedkv
+    inp = _small(B=1, H=64, q_lens=[T], kv_lens=[T], K=0, scenario=2, ratio=32, bs=16, D=D, win=40)
+    inp.ori_bt[0, 2::5] = -1
+    inp.cmp_bt[0, 0] = -1
+    d = inp.to("cuda")
+    kw = d.api_kwargs()
+    q = d.q.clone()
+    hit = [t for t in range(T) if t % 3 == 0 or t % 5 == 0]   # runs of 3 and of 5 tokens on 256 CUs
+    q[hit, 0, :] = float("nan")
+    q[hit[::2], 0, :] = float("inf")
+    ok = [t for t in range(T) if t not in set(hit)]
+    res = []
+    for qq in (d.q, q):
+        pc = prepare_sparse_attn_sharedkv(qq, **kw)
+        pc.launch()
+        torch.cuda.synchronize()
+        res.append((pc.out[ok].cpu(), pc.lse[ok].cpu()))
+    assert torch.isfinite(res[0][0].float()).all()
+    assert torch.equal(res[1][0], res[0][0]) and torch.equal(res[1][1], res[0][1])
