@@ -241,16 +241,17 @@ __global__ void __launch_bounds__(256) sas_fwd_win_kernel(const FwdParams p, con
 #pragma unroll
       for (int i = 0; i < 8; ++i) m = fmaxf(m, fmaxf(fmaxf(s[i][0], s[i][1]), fmaxf(s[i][2], s[i][3])));
       m = fmaxf(rows_max(m), sink2);
+      const float mb = m == -INFINITY ? 0.f : m;           // no sink and no row present: every P is 0
       float l = 0.f;
       uint32_t pk[8][2];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) { s[i][j] = __builtin_amdgcn_exp2f(s[i][j] - m); l += s[i][j]; }
+        for (int j = 0; j < 4; ++j) { s[i][j] = __builtin_amdgcn_exp2f(s[i][j] - mb); l += s[i][j]; }
         pk[i][0] = pack2<QT>(s[i][0], s[i][1]);
         pk[i][1] = pack2<QT>(s[i][2], s[i][3]);
       }
-      l = rows_sum(l) + __builtin_amdgcn_exp2f(sink2 - m);
+      l = rows_sum(l) + __builtin_amdgcn_exp2f(sink2 - mb);
       // O^T[channel][head] += V^T . P^T over 32 keys at a time
       f32x4 acc[NT];
 #pragma unroll
@@ -489,11 +490,12 @@ __global__ void __launch_bounds__(256, 2) sas_fwd_dense_kernel(const FwdParams p
           asm volatile("v_mul_f32 %0, %4, %0\n\tv_mul_f32 %1, %4, %1\n\tv_mul_f32 %2, %4, %2\n\tv_mul_f32 %3, %4, %3"
                        : "+v"(acc[i][0]), "+v"(acc[i][1]), "+v"(acc[i][2]), "+v"(acc[i][3]) : "v"(al));
       }
+      const float mb = m == -INFINITY ? 0.f : m;           // no sink and no row present yet: every P is 0
       uint32_t pk[4];
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) { s[mt][j] = __builtin_amdgcn_exp2f(s[mt][j] - m); l += s[mt][j]; }
+        for (int j = 0; j < 4; ++j) { s[mt][j] = __builtin_amdgcn_exp2f(s[mt][j] - mb); l += s[mt][j]; }
         pk[2 * mt] = pack2<QT>(s[mt][0], s[mt][1]);
         pk[2 * mt + 1] = pack2<QT>(s[mt][2], s[mt][3]);
       }
@@ -530,8 +532,8 @@ __global__ void __launch_bounds__(256, 2) sas_fwd_dense_kernel(const FwdParams p
       softmax_pv();
     }
     load_q(tn);
-    l = rows_sum(l) + __builtin_amdgcn_exp2f(sink2 - m);
-    store_out<PT, QT>(acc, 1.f / l, stage[wave], ob, lane);
+    l = rows_sum(l) + __builtin_amdgcn_exp2f(sink2 - (m == -INFINITY ? 0.f : m));
+    store_out<PT, QT>(acc, l == 0.f ? 0.f : 1.f / l, stage[wave], ob, lane);   // (0: no sink, no row)
     if (g == 0) lse[c16] = m * kLn2 + logf(l);
   }
   wait_vm<0>();   // the spare steps' DMA

@@ -927,3 +927,41 @@ def test_dense_runs_missing_rows_beside_a_non_finite_query(D, T):
         res.append((pc.out[ok].cpu(), pc.lse[ok].cpu()))
     assert torch.isfinite(res[0][0].float()).all()
     assert torch.equal(res[1][0], res[0][0]) and torch.equal(res[1][1], res[0][1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,spec", [
+    ("dense", dict(H=64, q_lens=[1040], kv_lens=[1040], scenario=2, ratio=32, D=512, win=63)),
+    ("dense_d576", dict(H=64, q_lens=[2060], kv_lens=[2060], scenario=2, ratio=32, win=63)),
+    ("window", dict(H=64, q_lens=[600], kv_lens=[600], scenario=1, win=31)),
+    ("window_d512", dict(H=16, q_lens=[900], kv_lens=[900], scenario=1, win=40, D=512)),
+])
+def test_runs_without_a_sink_and_with_missing_rows(name, spec):
+    """Sinks of -inf (no sink) over tokens whose first rows, or all of them, are
+    missing: the run kernels give what the one-workgroup-per-token kernel does
+    (a token without any row: an LSE of -inf, and 0 / 0 or zeros)."""
+    from dsv4_amd.api import prepare_sparse_attn_sharedkv
+    inp = _small(B=1, K=0, **spec)
+    inp.sinks[::2] = -float("inf")
+    inp.ori_bt[0, 2::3] = -1
+    if spec["scenario"] == 2:
+        inp.cmp_bt[0, :] = -1   # 64 rows a block, at most 64 of them: the window's rows alone remain
+    d = inp.to("cuda")
+    kw = d.api_kwargs()
+    res = []
+    for hw in (0, 4 if spec["scenario"] == 2 else 1):
+        pc = prepare_sparse_attn_sharedkv(d.q, head_waves=hw, **kw)
+        pc.out.fill_(float("nan"))
+        pc.launch()
+        torch.cuda.synchronize()
+        res.append((pc.out.float().cpu(), pc.lse.cpu()))
+    (o0, l0), (o1, l1) = res
+    assert not torch.isnan(l1).any() and torch.isinf(l1).any()
+    assert torch.equal(torch.isinf(l0), torch.isinf(l1))
+    fin = torch.isfinite(l1)
+    torch.testing.assert_close(l0[fin], l1[fin], atol=2e-5, rtol=2e-6)
+    assert torch.equal(torch.isnan(o0), torch.isnan(o1)) and torch.isfinite(o0[fin]).all()
+    o0, o1 = o0[fin], o1[fin]
+    step = 2.0 ** -8
+    assert float((o0 - o1).abs().max()) <= 2 * step * float(inp.ori_kv.abs().max())
+    assert float((o0 - o1).norm() / o1.norm()) < step
