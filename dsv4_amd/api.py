@@ -783,13 +783,16 @@ def _run_cached(r: _Cached, stream, dev, q, ori_kv, cmp_kv, cmp_sparse_indices, 
                 kv = base
             base += 4 * t.numel()
     try:
-        ws = _workspace(dev, stream, r.ws_bytes).data_ptr() if r.ws_bytes else 0
+        # held until the launch has been queued: nothing else may own it (under
+        # capture), or another thread may outgrow and replace the shared one
+        ws = _workspace(dev, stream, r.ws_bytes) if r.ws_bytes else None
         cmp_ = cmp_kv is not None
         rc = _fwd_bytes()(
             _PTRS.pack(q.data_ptr(), ori_kv.data_ptr(), ori_block_table.data_ptr(), cmp_kv.data_ptr() if cmp_ else 0,
                        cmp_block_table.data_ptr() if cmp_ else 0,
                        cmp_sparse_indices.data_ptr() if cmp_ and cmp_sparse_indices is not None else 0,
-                       cu, 0, kv, sinks.data_ptr(), out.data_ptr(), lse.data_ptr(), ws, r.ws_bytes) + r.tail, stream)
+                       cu, 0, kv, sinks.data_ptr(), out.data_ptr(), lse.data_ptr(),
+                       0 if ws is None else ws.data_ptr(), r.ws_bytes) + r.tail, stream)
         if rc:
             _lib.check(rc, "sparse_attn_sharedkv")
     finally:

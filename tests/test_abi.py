@@ -171,3 +171,31 @@ def test_bwd_rejects_both_window_modes_and_fwd_rejects_bwd_flags():
     for fl in (_lib.SAS_BWD_WINDOW_TOKENS, _lib.SAS_BWD_WINDOW_KEYS):
         rc, _, _ = _plan(_valid_args(flags=fl))
         assert rc == _lib.SAS_EINVAL and "flags" in _lib.lib().sas_last_error().decode()
+
+
+def test_cached_call_holds_its_workspace(monkeypatch):
+    """A cached call's workspace lives until its launch has been queued, also
+    when nothing else owns it (a captured call's, or a shared one outgrown by
+    another thread meanwhile)."""
+    import weakref
+    import torch
+    from dsv4_amd import api
+    r = object.__new__(api._Cached)
+    r.out_shape, r.lse_shape, r.tail, r.ws_bytes, r.host_names, r.B = (1, 16, 512), (1, 16), b"", 4096, [], 1
+    owned, launched = [], []
+
+    def workspace(dev, stream, nbytes):
+        t = torch.empty(nbytes, dtype=torch.uint8)
+        owned.append((weakref.ref(t), t.data_ptr()))
+        return t
+
+    def launch(packed, stream):
+        ptrs = api._PTRS.unpack(packed)
+        launched.append(owned[0][0]() is not None and ptrs[-2:] == (owned[0][1], 4096))
+        return 0
+
+    monkeypatch.setattr(api, "_workspace", workspace)
+    monkeypatch.setattr(api, "_fwd_bytes", lambda: launch)
+    q, row, i32 = torch.zeros(1, 16, 512), torch.zeros(1, 16, 1, 512), torch.zeros(2, dtype=torch.int32)
+    api._run_cached(r, 0, q.device, q, row, None, None, i32, None, i32, i32, torch.zeros(16), True)
+    assert launched == [True]
