@@ -867,8 +867,8 @@ def _prepare_backward(dout, q, out, lse, own_dq: bool, **kwargs) -> PreparedBack
     cmp_kv = kwargs.get("cmp_kv")
     keep = [dout_f, out_f, lse_f]
     direct, ws = C.c_int32(0), C.c_size_t(0)
-    _lib.check(_lib.lib().sas_bwd_plan(C.byref(_lib.SasBwdArgs(fwd=a)), C.byref(direct), C.byref(ws)),
-               "sparse_attn_sharedkv_backward")
+    _lib.check(_lib.lib().sas_bwd_plan(C.byref(_lib.SasBwdArgs(fwd=a, dout=dout_f.data_ptr())), C.byref(direct),
+                                       C.byref(ws)), "sparse_attn_sharedkv_backward")
     if ws.value:
         work = torch.empty(ws.value, dtype=torch.uint8, device=dev)
         keep.append(work)

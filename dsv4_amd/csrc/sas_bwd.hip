@@ -883,8 +883,12 @@ struct PrePlan {
   long long seg_groups, cmp_tiles, win_tiles;
   size_t ws;
 };
-PrePlan plan_prefill(const SasFwdArgs* a) {
+PrePlan plan_prefill(const SasBwdArgs* ba) {
+  const SasFwdArgs* a = &ba->fwd;
   PrePlan r{};
+  // q and dO reach LDS by DMA, 16 bytes a lane; the per-token kernels and the
+  // window pass load them through registers, at any alignment
+  if ((reinterpret_cast<uintptr_t>(a->q) | reinterpret_cast<uintptr_t>(ba->dout)) & 15) return r;
   const long long nslots = (long long)a->win_left + 1 + (a->scenario >= SAS_CFA ? a->K : 0);
   r.on = a->H % 32 == 0 && !(a->flags & SAS_BWD_WINDOW_TOKENS) && a->num_splits <= 0 &&
          ((a->flags & SAS_BWD_WINDOW_KEYS) || a->T >= 64 * a->B);
@@ -1040,7 +1044,7 @@ extern "C" int sas_bwd_v1(const SasBwdArgs* ba, void* stream) {
   if ((a->flags & SAS_BWD_WINDOW_TOKENS) && (a->flags & SAS_BWD_WINDOW_KEYS))
     return set_error(SAS_EINVAL, "bwd: SAS_BWD_WINDOW_TOKENS and SAS_BWD_WINDOW_KEYS together");
   const bool direct = a->flags & SAS_BWD_DQ_DTYPE, have_ws = a->flags & SAS_BWD_WORKSPACE;
-  const PrePlan pre = plan_prefill(a);
+  const PrePlan pre = plan_prefill(ba);
   if (direct && !(pre.on && have_ws))
     return set_error(SAS_EINVAL, "bwd: SAS_BWD_DQ_DTYPE without SAS_BWD_WORKSPACE or where sas_bwd_plan does not allow it");
   if (have_ws && pre.on && (!a->workspace || a->workspace_bytes < pre.ws))
@@ -1128,7 +1132,7 @@ extern "C" int sas_bwd_plan(const SasBwdArgs* ba, int32_t* dq_dtype, size_t* wor
   using namespace sas;
   clear_error();
   if (!ba) return set_error(SAS_EINVAL, "bwd: null args");
-  const PrePlan pre = ba->fwd.T >= 0 && ba->fwd.B >= 1 && ba->fwd.H >= 1 ? plan_prefill(&ba->fwd) : PrePlan{};
+  const PrePlan pre = ba->fwd.T >= 0 && ba->fwd.B >= 1 && ba->fwd.H >= 1 ? plan_prefill(ba) : PrePlan{};
   if (dq_dtype) *dq_dtype = pre.on;
   if (workspace_bytes) *workspace_bytes = pre.ws;
   return SAS_OK;

@@ -261,8 +261,9 @@ typedef struct SasBwdArgs {
 int sas_bwd_v1(const SasBwdArgs* a, void* stream);
 
 /* Whether these arguments may set SAS_BWD_DQ_DTYPE, and the workspace bytes of
-   SAS_BWD_WORKSPACE (0: none is used). Reads dims, scenario, num_splits and the
-   window flags only. */
+   SAS_BWD_WORKSPACE (0: none is used). Reads dims, scenario, num_splits, the
+   window flags and whether q and dout are 16-byte aligned (the prefill path
+   takes no others). */
 int sas_bwd_plan(const SasBwdArgs* a, int32_t* dq_dtype, size_t* workspace_bytes);
 
 /*

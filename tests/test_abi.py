@@ -199,3 +199,16 @@ def test_cached_call_holds_its_workspace(monkeypatch):
     q, row, i32 = torch.zeros(1, 16, 512), torch.zeros(1, 16, 1, 512), torch.zeros(2, dtype=torch.int32)
     api._run_cached(r, 0, q.device, q, row, None, None, i32, None, i32, i32, torch.zeros(16), True)
     assert launched == [True]
+
+
+@pytest.mark.parametrize("q,dout,on", [(4096, 8192, 1), (4096, 8200, 0), (4098, 8192, 0), (None, None, 1)])
+def test_backward_plan_asks_for_aligned_rows(q, dout, on):
+    """The prefill path moves q and dout 16 bytes a lane: other alignments
+    keep the kernels that load them through registers, on the host's word
+    alone (with SAS_BWD_DQ_DTYPE the call is then refused)."""
+    a = _valid_args(T=128, B=1, H=64)
+    a.q = q
+    dq, ws = C.c_int32(-1), C.c_size_t(1)
+    ba = _lib.SasBwdArgs(fwd=a, dout=dout)
+    assert _lib.lib().sas_bwd_plan(C.byref(ba), C.byref(dq), C.byref(ws)) == 0
+    assert dq.value == on and (ws.value > 0) == bool(on)

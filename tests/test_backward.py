@@ -654,3 +654,29 @@ def test_gpu_backward_non_finite_token_stays_in_its_rows(spec, what):
         assert float((a[free] - b[free]).abs().max()) <= 1e-5 * float(b[free].abs().max()), name
     snk = got[3][heads]
     assert torch.isfinite(snk).all()
+
+
+@pytest.mark.gpu
+def test_gpu_backward_output_gradient_at_any_alignment():
+    """An output gradient that starts 8 bytes off a 16-byte boundary: the
+    gradients of the aligned one, by the kernels that load it through
+    registers."""
+    from dsv4_amd import _lib
+    from dsv4_amd.api import prepare_sparse_attn_sharedkv_backward, sparse_attn_sharedkv, sparse_attn_sharedkv_backward
+    from tests.test_gpu_parity import _small
+    inp = _small(B=1, H=64, q_lens=[130], kv_lens=[300], K=24)
+    d = inp.to("cuda")
+    kw = d.api_kwargs()
+    out, lse = sparse_attn_sharedkv(d.q, return_softmax_lse=True, **kw)
+    g = torch.Generator().manual_seed(53)
+    dout = torch.randn(out.shape, generator=g).to(out.dtype)
+    buf = torch.zeros(dout.numel() + 4, dtype=dout.dtype, device="cuda")
+    off = buf[4:].view(dout.shape)
+    off.copy_(dout)
+    assert off.data_ptr() % 16 == 8 and off.is_contiguous()
+    r = _oracle_bwd(inp, dout, out, lse)
+    pb = prepare_sparse_attn_sharedkv_backward(off, d.q, out, lse, **kw)
+    assert not pb.args.fwd.flags & _lib.SAS_BWD_WORKSPACE
+    got = sparse_attn_sharedkv_backward(off, d.q, out, lse, **kw)
+    torch.cuda.synchronize()
+    _check_against_oracle("dout off alignment", inp, *got, r)
