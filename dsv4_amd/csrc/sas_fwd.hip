@@ -2072,15 +2072,27 @@ int make_plan(const SasFwdArgs* a, Plan* pl) {
   return SAS_OK;
 }
 
-// Window-only calls walk runs of tokens (sas_fwd_win.hip) once one workgroup
-// per (token, head group) would take more than one round of the CUs. Below
-// that the run's first window costs more than it saves (64 heads, D = 576:
-// 128 tokens 15.2 against 14.4 us, 256 tokens 17.3 against 16.2, 384 tokens
-// 21.6 against 27.4, 1000 tokens 39 against 55; 16 heads, 1500 tokens 22
-// against 66).
-bool win_runs(const SasFwdArgs* a, const Plan& pl) {
-  return pl.exact && a->scenario == SAS_SWA && a->kv_dtype == a->q_dtype && a->win_left < 128 &&
-         a->head_waves == 0 && (long long)a->T * pl.nhg > sas::device_cus();
+// Window-only calls walk runs of tokens (sas_fwd_win.hip): the tokens of a run,
+// or 0 for one workgroup per (token, head group). A run belongs to one sequence:
+// a sequence of the mean length is cut into as many equal runs as leave all
+// sequences' in one round of the CUs, or stays whole (140 sequences of 3 tokens,
+// 64 heads: runs of 3 tokens 28.7 us, of ceil(T / CUs) = 2 tokens 44.0). Runs
+// are taken where their rounds cost less: a round of them loads a whole window
+// and then works through `units` (16 heads of a token) a wave, about 0.75 + 0.4
+// units of the other kernel's round. H = 64, D = 576, per token against runs:
+// one sequence of 256 / 384 / 1000 tokens 16.2 / 27.4 / 55 against 17.3 / 21.6 /
+// 39 us; 300 / 1024 sequences of one token 31 / 79 against 35 / 104 us (128
+// heads 44 / 144 against 46 / 130, 48 heads 49 / 159 against 33 / 99); of one or
+// two 35 / 126 against 41 / 112; of two 49 / 163 against 47 / 128.
+int win_run(const SasFwdArgs* a, const Plan& pl) {
+  if (!pl.exact || a->scenario != SAS_SWA || a->kv_dtype != a->q_dtype || a->win_left >= 128 || a->head_waves != 0)
+    return 0;
+  const long long cus = sas::device_cus(), len = std::max<long long>(1, a->T / a->B);
+  const long long per_seq = std::max<long long>(1, cus / a->B);
+  const long long run = std::min<long long>(kRunTokens, std::max((len + per_seq - 1) / per_seq, (a->T + cus - 1) / cus));
+  const long long rounds = (a->B * ((len + run - 1) / run) + cus - 1) / cus;
+  const double units = std::max(1.0, std::min((double)run, (double)a->T / a->B) * a->H / 64);
+  return (a->T * pl.nhg + cus - 1) / cus > rounds * (0.75 + 0.4 * units) ? (int)run : 0;
 }
 
 // Dense compressed calls walk runs of tokens too, from four (D = 512) or eight
@@ -2250,12 +2262,12 @@ extern "C" int sas_fwd_v1(const SasFwdArgs* a, void* stream) {
   fp.out_nt = pl.nsplit == 1 && (size_t)a->T * a->H * kDV * 2 >= (size_t(16) << 20);
   hipStream_t st = (hipStream_t)stream;
 
-  if (win_runs(a, pl) || dense_runs(a, pl)) {
+  if (const int run = win_run(a, pl)) return launch_fwd_win(fp, (int)a->D, a->q_dtype, run, st);
+  if (dense_runs(a, pl)) {
     // (two dense workgroups share a CU)
-    const bool cfa = a->scenario == SAS_CFA;
-    const long long cus = (cfa ? 2LL : 1LL) * sas::device_cus(), per = cfa ? a->H / 64 : 1;
+    const long long cus = 2LL * sas::device_cus(), per = a->H / 64;
     fp.nhg = (int)per;
-    return launch_fwd_win(fp, (int)a->D, a->q_dtype, (int)std::min<long long>(64, (a->T * per + cus - 1) / cus), st);
+    return launch_fwd_win(fp, (int)a->D, a->q_dtype, (int)std::min<long long>(kRunTokens, (a->T * per + cus - 1) / cus), st);
   }
   if (fp8) rc = dispatch_hw<576, __bf16, 1>(pl.hw, pl.nw, pl.exact, fp, nblocks, st);
   else if (a->q_dtype == SAS_DT_BF16)

@@ -965,3 +965,41 @@ def test_runs_without_a_sink_and_with_missing_rows(name, spec):
     step = 2.0 ** -8
     assert float((o0 - o1).abs().max()) <= 2 * step * float(inp.ori_kv.abs().max())
     assert float((o0 - o1).norm() / o1.norm()) < step
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,spec,runs", [
+    # one workgroup per token: sequences of one token; one round of them
+    ("one_token_h64", dict(B=300, H=64, q_lens=[1] * 300, kv_lens=[60 + i for i in range(300)]), False),
+    ("one_token_h16_d512", dict(B=300, H=16, q_lens=[1] * 300, kv_lens=[140] * 300, D=512), False),
+    ("one_round", dict(B=2, H=64, q_lens=[200, 56], kv_lens=[200, 300]), False),
+    # runs: one-token sequences of many head groups, whole short sequences,
+    # sequences around and beyond the mean length, a padded empty one
+    ("one_token_h48", dict(B=260, H=48, q_lens=[1] * 260, kv_lens=[130] * 260), True),
+    ("whole_sequences", dict(B=140, H=64, q_lens=[3] * 140, kv_lens=[90] * 140, D=512), True),
+    ("ragged", dict(B=9, H=32, q_lens=[1, 250, 0, 17, 18, 19, 2, 90, 33], kv_lens=[200, 250, 9, 17, 90, 300, 1, 95, 40], bs=16), True),
+])
+def test_window_run_rule(name, spec, runs):
+    """The rule between runs of tokens and one workgroup per token, on both
+    sides of it: the per-token kernel's results (head_waves given; the same
+    bits where the rule keeps that kernel and its head groups)."""
+    from dsv4_amd.api import prepare_sparse_attn_sharedkv
+    inp = _small(K=0, scenario=1, **spec)
+    d = inp.to("cuda")
+    kw = d.api_kwargs()
+    hw = 4 if spec["H"] % 64 == 0 else 2 if spec["H"] % 32 == 0 else 1
+    res = []
+    for h in (0, hw):
+        pc = prepare_sparse_attn_sharedkv(d.q, head_waves=h, **kw)
+        pc.out.fill_(float("nan"))
+        pc.launch()
+        torch.cuda.synchronize()
+        res.append((pc.out.float().cpu(), pc.lse.cpu()))
+    (o0, l0), (o1, l1) = res
+    assert torch.isfinite(o0).all()
+    torch.testing.assert_close(l0, l1, atol=2e-5, rtol=2e-6)
+    # a P moves by at most one rounding step (2^-8 in bf16)
+    assert float((o0 - o1).abs().max()) <= 2.0 ** -8 * float(inp.ori_kv.abs().max())
+    assert float((o0 - o1).norm() / o1.norm()) < 2.0 ** -8
+    if not runs:
+        assert torch.equal(o0, o1) and torch.equal(l0, l1)
