@@ -29,6 +29,7 @@ Device ``cu_seqlens_q`` is passed to the kernel as it is.
 from __future__ import annotations
 
 import ctypes as C
+import itertools
 import struct
 import threading
 from collections import OrderedDict
@@ -619,7 +620,8 @@ def prepare_sparse_attn_sharedkv(
 # ---------------------------------------------------------------------------
 
 _CACHE_MAX = 64
-_cache: "OrderedDict[tuple, _Cached]" = OrderedDict()
+_cache: "dict[tuple, _Cached]" = {}   # the least recently used one leaves (by _Cached.used)
+_uses = itertools.count()
 _cache_lock = threading.Lock()
 
 
@@ -705,6 +707,7 @@ def sparse_attn_sharedkv(
     dev = q.device
     stream = _raw_stream(dev) if q.is_cuda else None
     if r is not None:
+        r.used = next(_uses)
         return _run_cached(r, stream, dev, q, ori_kv, cmp_kv, cmp_sparse_indices, ori_block_table, cmp_block_table,
                            cu_seqlens_q, seqused_kv, sinks, return_softmax_lse)
     r = _resolve(q, ori_kv=ori_kv, cmp_kv=cmp_kv, cmp_sparse_indices=cmp_sparse_indices,
@@ -719,7 +722,7 @@ def sparse_attn_sharedkv(
         with _cache_lock:
             _cache[key] = kept
             if len(_cache) > _CACHE_MAX:
-                _cache.popitem(last=False)
+                del _cache[min(_cache.items(), key=lambda kv: kv[1].used)[0]]
     out = torch.empty((r.T1, r.N1, 512), dtype=r.dtype, device=dev)
     lse = torch.empty((r.T1, r.N1), dtype=torch.float32, device=dev)
     a = _lib.SasFwdArgs.from_buffer_copy(r.args)
@@ -749,7 +752,7 @@ class _Cached:
     """What a signature's later calls need of its resolution: no tensor, no
     address (TND calls whose operands are used as given)."""
 
-    __slots__ = ("out_shape", "lse_shape", "tail", "ws_bytes", "host_names", "B")
+    __slots__ = ("out_shape", "lse_shape", "tail", "ws_bytes", "host_names", "B", "used")
 
     def __init__(self, r: _Resolved):
         self.out_shape, self.lse_shape = (r.T1, r.N1, 512), (r.T1, r.N1)
@@ -757,6 +760,7 @@ class _Cached:
         self.ws_bytes = r.ws_bytes
         self.host_names = [name for name, _ in r.host_parts]
         self.B = r.B
+        self.used = next(_uses)
 
 
 def _run_cached(r: _Cached, stream, dev, q, ori_kv, cmp_kv, cmp_sparse_indices, ori_block_table, cmp_block_table,

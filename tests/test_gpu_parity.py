@@ -1003,3 +1003,27 @@ def test_window_run_rule(name, spec, runs):
     assert float((o0 - o1).norm() / o1.norm()) < 2.0 ** -8
     if not runs:
         assert torch.equal(o0, o1) and torch.equal(l0, l1)
+
+
+@pytest.mark.gpu
+def test_signature_in_use_is_kept(monkeypatch):
+    """A signature called all along outlives any number of others (the cache
+    drops the one least recently used)."""
+    from dsv4_amd import api
+    inp = _small(B=1, H=16, q_lens=[api._CACHE_MAX + 40], kv_lens=[600], K=16).to("cuda")
+    kw = inp.api_kwargs()
+
+    def call(n):
+        k = dict(kw, cu_seqlens_q=torch.tensor([0, n], dtype=torch.int32), cmp_sparse_indices=inp.cmp_idx[:n])
+        api.sparse_attn_sharedkv(inp.q[:n], **k)
+
+    call(1)
+    resolved = []
+    real = api._resolve
+    monkeypatch.setattr(api, "_resolve", lambda q, **k: (resolved.append(q.shape[0]), real(q, **k))[1])
+    for n in range(2, api._CACHE_MAX + 40):
+        call(n)
+        call(1)
+    torch.cuda.synchronize()
+    assert 1 not in resolved and len(resolved) == api._CACHE_MAX + 38
+    assert len(api._cache) <= api._CACHE_MAX
