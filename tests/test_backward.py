@@ -174,6 +174,7 @@ def _check_elem(got, ref, what, tol=GRAD_TOL):
     ratio = err / bound.clamp_min(1e-300)
     bad = err > bound
     worst = float(ratio.max())
+    assert bool(torch.isfinite(got).all()), f"{what}: {int((~torch.isfinite(got)).sum())} non-finite elements"
     assert not bool(bad.any()), (f"{what}: {int(bad.sum())} of {err.numel()} elements beyond "
                                  f"{tol}|ref| + {tol} rowmax|ref| (worst err/bound {worst:.3g})")
     return worst
@@ -302,12 +303,12 @@ def test_gpu_backward_c3_prefill_sampled():
 @pytest.mark.parametrize("name", ["prefill_2b", "prefill_bs16_h16", "swa", "short_kv", "decode_h64", "cfa",
                                   "fp16_d512", "prefill_wide_window", "prefill_swa_bs16"])
 def test_gpu_backward_window_pass_both_ways(name):
-    """Window rows' gradients summed per (token, row) and by the key-major
-    window pass (forced both ways, whatever the library would choose): each
-    element-wise against the fp64 oracle, on prefills (several batches, BSND
-    pages of 16, a window wider than the 64-position tile) and on
-    decode and short-KV batches (tokens with empty windows, rows past
-    act_kv)."""
+    """Rows' gradients summed per (token, row) and key-major (forced both ways,
+    whatever the library would choose: all rows by the prefill path where H is
+    a multiple of 32, the window rows by the window pass elsewhere): each
+    element-wise against the fp64 oracle, on prefills (several batches, pages
+    of 16, a window wider than the 64-position tile) and on decode and
+    short-KV batches (tokens with empty windows, rows past act_kv)."""
     from dsv4_amd.api import sparse_attn_sharedkv, sparse_attn_sharedkv_backward
     from tests.test_gpu_parity import _small
     extra = {
@@ -331,9 +332,9 @@ def test_gpu_backward_window_pass_both_ways(name):
 
 @pytest.mark.gpu
 def test_gpu_backward_window_pass_bsnd():
-    """The key-major window pass with BSND queries (per-batch lengths, padded
-    rows: the kernel reads act_q instead of a prefix difference) gives the
-    TND per-token result up to summation order."""
+    """The key-major passes with BSND queries (per-batch lengths, padded rows:
+    the kernels read act_q instead of a prefix difference) give the TND
+    per-token result up to summation order."""
     from tests.test_gpu_parity import _small
     from dsv4_amd.api import sparse_attn_sharedkv, sparse_attn_sharedkv_backward
     q_lens = [70, 30]
@@ -367,13 +368,12 @@ def test_gpu_backward_window_pass_bsnd():
 
 @pytest.mark.gpu
 def test_gpu_backward_captured_in_a_graph():
-    """The backward of a prefill captured in a HIP graph: eagerly the window
-    pass runs beside the per-token kernel on the library's side stream;
-    under capture it either gives way to per-token adds (the default) or,
-    when asked for, runs after the per-token kernel on the captured stream.
+    """The prepared backward of a prefill captured in a HIP graph: with its fp32
+    dq it gives way to per-token adds under capture (the default) or, when
+    asked for, sums every row's gradient key-major on the captured stream.
     Every replay (with eager work between them) equals the eager run of the
     same mode up to fp32 summation order; the two modes differ from each
-    other only by where the window keys' products are rounded."""
+    other only by where the keys' products are rounded."""
     from dsv4_amd.api import prepare_sparse_attn_sharedkv_backward, sparse_attn_sharedkv
     from tests.test_gpu_parity import _small
     inp = _small(B=2, H=64, q_lens=[300, 170], kv_lens=[300, 420], K=64)
@@ -680,3 +680,116 @@ def test_gpu_backward_output_gradient_at_any_alignment():
     got = sparse_attn_sharedkv_backward(off, d.q, out, lse, **kw)
     torch.cuda.synchronize()
     _check_against_oracle("dout off alignment", inp, *got, r)
+
+
+# ---------------------------------------------------------------------------
+# callers without a workspace: per-token kernels, the window pass beside them
+# ---------------------------------------------------------------------------
+
+def _without_workspace(pb):
+    """A prepared backward as a C caller that gives no workspace calls it."""
+    from dsv4_amd import _lib
+    a = pb.args.fwd
+    a.flags &= ~_lib.SAS_BWD_WORKSPACE
+    a.workspace, a.workspace_bytes = None, 0
+    return pb
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,spec", [
+    # the 64-head and the 32-head per-token kernel, prefills (the window pass
+    # beside them on the library's side stream) and decode-like calls
+    ("h64", dict(B=2, H=64, q_lens=[300, 170], kv_lens=[300, 420], K=64)),
+    ("h128_d512_fp16", dict(B=1, H=128, q_lens=[140], kv_lens=[500], K=48, D=512, dtype=torch.float16)),
+    ("h32_bs16", dict(B=3, H=32, q_lens=[90, 17, 130], kv_lens=[90, 200, 130], K=32, bs=16)),
+    ("h32_wide_window", dict(B=1, H=32, q_lens=[200], kv_lens=[400], K=48, win=300)),
+    ("h64_swa", dict(B=2, H=64, q_lens=[200, 70], kv_lens=[260, 70], K=0, scenario=1)),
+    ("h64_cfa", dict(B=2, H=64, q_lens=[128, 40], kv_lens=[500, 40], K=0, scenario=2, ratio=8)),
+    ("h64_short_kv", dict(B=2, H=64, q_lens=[150, 90], kv_lens=[40, 3], K=8)),
+    ("h64_decode", dict(B=3, H=64, q_lens=[1, 2, 1], kv_lens=[700, 90, 300], K=64)),
+])
+def test_gpu_backward_without_workspace(name, spec):
+    """Without a workspace: the library's choice, per-token adds for every row,
+    and the window pass, each element-wise against the fp64 oracle."""
+    from dsv4_amd.api import prepare_sparse_attn_sharedkv_backward, sparse_attn_sharedkv
+    from tests.test_gpu_parity import _small
+    inp = _small(**spec)
+    d = inp.to("cuda")
+    kw = d.api_kwargs()
+    out, lse = sparse_attn_sharedkv(d.q, return_softmax_lse=True, **kw)
+    g = torch.Generator().manual_seed(59)
+    dout = torch.randn(out.shape, generator=g).to(inp.q.dtype)
+    r = _oracle_bwd(inp, dout, out, lse)
+    dout = dout.cuda()
+    for wp in (None, False, True):
+        pb = _without_workspace(prepare_sparse_attn_sharedkv_backward(dout, d.q, out, lse, window_pass=wp, **kw))
+        pb.launch()
+        torch.cuda.synchronize()
+        _check_against_oracle(f"{name} no workspace window_pass={wp}", inp, *pb.result(), r)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H", [32, 64])
+def test_gpu_backward_without_workspace_captured(H):
+    """The same under capture: per-token adds (the default), or the window pass
+    after the per-token kernel on the captured stream, on every replay."""
+    from dsv4_amd.api import prepare_sparse_attn_sharedkv_backward, sparse_attn_sharedkv
+    from tests.test_gpu_parity import _small
+    inp = _small(B=2, H=H, q_lens=[200, 70], kv_lens=[200, 320], K=32)
+    d = inp.to("cuda")
+    kw = d.api_kwargs()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        out, lse = sparse_attn_sharedkv(d.q, return_softmax_lse=True, **kw)
+        g = torch.Generator().manual_seed(61)
+        dout = torch.randn(out.shape, generator=g).to(inp.q.dtype)
+        r = _oracle_bwd(inp, dout, out, lse)
+        dout = dout.cuda()
+        for wp in (None, True):
+            pb = _without_workspace(prepare_sparse_attn_sharedkv_backward(dout, d.q, out, lse, window_pass=wp, **kw))
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=side):
+                pb.zero_grads()
+                pb.launch(side)
+            for i in range(3):
+                for t in (pb.dq, pb.d_ori_kv, pb.d_cmp_kv, pb.d_sinks):
+                    t.fill_(float(i + 7))             # eager work between replays
+                graph.replay()
+                torch.cuda.synchronize()
+                _check_against_oracle(f"captured H{H} window_pass={wp} replay {i}", inp, *pb.result(), r)
+            del graph, pb
+
+
+@pytest.mark.gpu
+def test_gpu_backward_without_workspace_bsnd():
+    """The window pass beside the per-token kernels with BSND queries (padded
+    rows, lengths read from act_q): the TND gradients up to summation order."""
+    from tests.test_gpu_parity import _small
+    from dsv4_amd.api import prepare_sparse_attn_sharedkv_backward, sparse_attn_sharedkv
+    q_lens, S = [130, 40], 130
+    inp = _small(B=2, H=64, q_lens=q_lens, kv_lens=[200, 40], K=16)
+    d = inp.to("cuda")
+    kw = d.api_kwargs()
+    out, lse = sparse_attn_sharedkv(d.q, return_softmax_lse=True, **kw)
+    g = torch.Generator().manual_seed(67)
+    dout = torch.randn(out.shape, generator=g).to(out.dtype).cuda()
+
+    def padded(t, fill=0):
+        p = torch.full((2, S) + tuple(t.shape[1:]), fill, dtype=t.dtype, device="cuda")
+        p[0], p[1, :40] = t[:130], t[130:]
+        return p
+
+    kwb = dict(kw, layout_q="BSND", cmp_sparse_indices=padded(d.cmp_idx, -1))
+    ref = prepare_sparse_attn_sharedkv_backward(dout, d.q, out, lse, window_pass=False, **kw)
+    pb = _without_workspace(prepare_sparse_attn_sharedkv_backward(padded(dout), padded(d.q), padded(out), padded(lse), **kwb))
+    ref.launch()
+    pb.launch()
+    torch.cuda.synchronize()
+    (dq, *rows), (dq_ref, *rows_ref) = pb.result(), ref.result()
+    assert _rel_err(dq[0].float().cpu(), dq_ref[:130].float().cpu()) < 1e-2
+    assert _rel_err(dq[1, :40].float().cpu(), dq_ref[130:].float().cpu()) < 1e-2
+    assert torch.count_nonzero(dq[1, 40:].cpu().float()) == 0
+    for a, b in zip(rows, rows_ref):
+        assert _rel_err(a.cpu(), b.cpu()) < 1e-4

@@ -699,8 +699,8 @@ def test_drop_in_call_captured_in_a_graph_keeps_its_workspace():
 
 def test_api_repeated_calls_read_current_values():
     """The drop-in call caches its argument resolution per signature
-    (shapes, dtypes, device addresses, scalars, stream): repeated calls must
-    still read the current values of every input. Host sequence lengths
+    (shapes, dtypes, devices, scalars): repeated calls must still read the
+    current values of every input. Host sequence lengths
     changed in place, device q / indices rewritten in place, and a fresh q
     tensor each give the oracle's result for the values at that call."""
     inp = _small(B=3, H=64, q_lens=[1, 2, 1], kv_lens=[900, 700, 300], K=64, seed=5)
@@ -846,6 +846,7 @@ def test_window_runs_bsnd_padding():
     ("limits", dict(B=1, H=64, q_lens=[1030], kv_lens=[1031], ratio=8, D=512, win=128)),
     ("ratio1_win1", dict(B=17, H=64, q_lens=[128] * 17, kv_lens=[128] * 17, ratio=1, win=0)),
     ("short_kv", dict(B=2, H=64, q_lens=[800, 300], kv_lens=[350, 3], ratio=4, win=40, D=512)),
+    ("short_kv_d576", dict(B=2, H=64, q_lens=[1700, 400], kv_lens=[700, 3], ratio=8, win=40)),
     ("missing_blocks", dict(B=1, H=128, q_lens=[1050], kv_lens=[1050], ratio=16, bs=16)),
 ])
 def test_dense_runs_match_per_token(name, spec):
@@ -882,12 +883,15 @@ def test_signature_cache_takes_new_buffers():
     """A call of a shape seen before on other buffers, from another stream and
     with other host lengths, reads its own operands (a resolution holds no
     address): equal to a freshly prepared call, for host and device lengths."""
+    from dsv4_amd import api
     from dsv4_amd.api import prepare_sparse_attn_sharedkv, sparse_attn_sharedkv
     side = torch.cuda.Stream()
+    api._cache.clear()
     for host in (True, False):
         for seed in range(3):
-            inp = _small(B=3, H=64, q_lens=[1, 2, 1], kv_lens=[900 + 40 * seed, 700, 333], K=48, seed=seed)
-            if seed == 2:   # the tables' width is part of the signature: keep it
+            # (lengths that keep the tables' width and the pool's size, both part of the signature)
+            inp = _small(B=3, H=64, q_lens=[1, 2, 1], kv_lens=[900 + 40 * min(seed, 1), 700, 333], K=48, seed=seed)
+            if seed == 2:
                 inp.seqused_kv[0] = 901
             d = inp.to("cuda")
             kw = d.api_kwargs()
@@ -901,6 +905,7 @@ def test_signature_cache_takes_new_buffers():
                     out, lse = sparse_attn_sharedkv(d.q, return_softmax_lse=True, **kw)
                 torch.cuda.synchronize()
                 assert torch.equal(out, ref.out) and torch.equal(lse, ref.lse), (host, seed)
+        assert len(api._cache) == (1 if host else 2)   # one signature for the host lengths, one for the device's
 
 
 @pytest.mark.gpu
