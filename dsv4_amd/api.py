@@ -686,8 +686,8 @@ def sparse_attn_sharedkv(
     # The signature is the tensors' geometry: what a resolution holds (checks,
     # dims, the split plan) depends on no address, so new buffers of a shape
     # seen before pay nothing extra. (With the addresses in it, and 9 helper
-    # calls to build it, a repeated 1-token call took the host 13.5 us and the
-    # first on new buffers 96 us.)
+    # calls to build it, a repeated 1-token call took the host 13.6-14.1 us and
+    # the first on new buffers 75-78; now 12.4 and 44-51.)
     key = (q.shape, q.dtype, q.get_device(), q.is_contiguous(),
            ori_kv.shape, ori_kv.dtype, ori_kv.get_device(), ori_kv.is_contiguous(),
            ori_block_table.shape, ori_block_table.dtype, ori_block_table.get_device(), ori_block_table.is_contiguous(),
@@ -832,12 +832,13 @@ def prepare_sparse_attn_sharedkv_backward(dout: torch.Tensor, q: torch.Tensor, o
                                           lse: torch.Tensor, **kwargs) -> PreparedBackward:
     """Validate and bind the arguments of :func:`sparse_attn_sharedkv_backward`
     and allocate its (zeroed) gradient buffers. ``window_pass`` (keyword,
-    default None: the library's choice, the key-major pass for prefills)
-    selects how window rows' gradients are summed: True, the key-major pass
-    (each row's gradient summed over the tokens whose window holds it, one
-    add per 16 heads, beside the per-token kernel on a side stream); False,
-    one add per (token, row); the results agree up to fp32 summation
-    order."""
+    default None: the library's choice, key-major for prefills) selects how
+    cache rows' gradients are summed: True, key-major (each row's gradient
+    summed over the tokens that attend it, one add per segment of tokens and
+    32 heads; where H is not a multiple of 32, or q or dout not 16-byte
+    aligned, the window rows alone, beside the per-token kernel on a side
+    stream); False, one add per (token, row). The results agree up to fp32
+    summation order."""
     return _prepare_backward(dout, q, out, lse, False, **kwargs)
 
 

@@ -569,7 +569,8 @@ __global__ void __launch_bounds__(512) sas_bwd64_kernel(const BwdParams bp) {
 // resolve(): position below act_kv, block inside the table, table entry
 // inside the cache. It runs beside the per-token kernel on a side stream
 // (SideStream below); sas_bwd_v1 chooses it for prefills that do not take the
-// prefill path (sas_bwd_pre.hip: no workspace given, or H not a multiple of 32).
+// prefill path (sas_bwd_pre.hip: no workspace given, H not a multiple of 32, or
+// q or dO not 16-byte aligned).
 constexpr int kWinRows = 64;   // positions per tile (16 per wave)
 
 template <int D, typename QT>

@@ -2095,10 +2095,9 @@ int win_run(const SasFwdArgs* a, const Plan& pl) {
   return (a->T * pl.nhg + cus - 1) / cus > rounds * (0.75 + 0.4 * units) ? (int)run : 0;
 }
 
-// Dense compressed calls walk runs of tokens too, from four (D = 512) or eight
-// (D = 576, whose two workgroups per CU spill a little) rounds of 64-head
-// workgroups on and where batches are long enough to have runs (64 heads,
-// ratio 128: D = 576, 512 tokens 32.6 against 28.0 us, 1000 tokens 50.6 against
+// Dense compressed calls walk runs of tokens too, where batches are long enough
+// to have runs and from four (D = 512) or eight (D = 576) rounds of 64-head
+// workgroups on: there the runs were measured faster (64 heads, ratio 128: D = 576, 512 tokens 32.6 against 28.0 us, 1000 tokens 50.6 against
 // 52.0, 2000 tokens 90 against 97, 3 x 301 tokens with 128 heads and a 64-row
 // window 86.8 against 86.1; D = 512 with 128 heads, 512 tokens 42 against 53;
 // 300 batches of 3 tokens 69 against 61).

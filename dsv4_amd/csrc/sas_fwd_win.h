@@ -1,4 +1,5 @@
-// Window-only forward over runs of consecutive tokens (sas_fwd_win.hip).
+// Window-only and dense compressed forward over runs of consecutive tokens
+// (sas_fwd_win.hip).
 #pragma once
 
 #include "sas_kern.h"

@@ -12,7 +12,7 @@
 // A wave's unit is (token, 16 heads), all keys and channels: S over the whole
 // window first, then P against the final maximum (as the exact schedule
 // rounds it), then P.V; the next unit's query is loaded under P.V. 8192 tokens,
-// 64 heads, D = 512: 247 us against 447 (copy-rate floor 210: query and
+// 64 heads, D = 512: 247 us against 406 (copy-rate floor 210: query and
 // output, 1.08 GB).
 
 #include "sas_fwd_win.h"
@@ -310,9 +310,9 @@ __global__ void __launch_bounds__(256) sas_fwd_win_kernel(const FwdParams p, con
 // when a row's maximum rises by more than 2^8. A step is ~4500 clk of mostly
 // serial work (scores 1200, softmax 1300, P.V 1350) and a token's output
 // stores another 5400, so two workgroups share each CU (80 KB of LDS and 256
-// registers a wave each): one, with four slots and a deeper DMA lead, took
-// 520 us for 8192 tokens, 64 heads, D = 512, ratio 128; two take 360, the
-// one-workgroup-per-token kernel 452.
+// registers a wave each, 14 to 17 of them spilled): one, with four slots and a
+// deeper DMA lead, took 520 us for 8192 tokens, 64 heads, D = 512, ratio 128;
+// two take 364, the one-workgroup-per-token kernel 452.
 __device__ const uint4 kZeroRow[576 * 2 / 16] = {};   // a missing row's bytes: finite, whatever the caller's hold
 
 template <int D, typename QT>
@@ -371,7 +371,7 @@ __global__ void __launch_bounds__(256, 2) sas_fwd_dense_kernel(const FwdParams p
     j = max(min(j, r.n - 1), 0);
     return tab[j < r.nwin ? r.wb + j : kDenseWinRows + j - r.nwin];
   };
-  // producer: step ps of token pt goes to slot pi % 4; a wave moves the rows
+  // producer: step ps of token pt goes to slot pi % 2; a wave moves the rows
   // 8 wave .. + 7 of every step in RI instructions
   int pt = rn.r0, ps = 0, pi = 0;
   Rows pr = rows_of(pt);

@@ -153,22 +153,26 @@ typedef struct SasFwdArgs {
 #define SAS_FWD_NO_COMBINE 1
 
 /* SasFwdArgs.flags of a sas_bwd_v1 call (the forward rejects them): how the
-   window rows' gradients are summed. SAS_BWD_WINDOW_TOKENS: one fp32 add per
-   (token, row, head group, channel). SAS_BWD_WINDOW_KEYS: a key-major pass
-   sums each window row's gradient over the tokens whose window holds it and
-   adds it once per 16-head group; it runs beside the per-token kernel on a
-   side stream of the library (one per device, created on first use, forked
-   from and joined back to `stream` by events; one after the other on
-   `stream` while it is being captured). Neither flag: the key-major pass for
-   calls with at least 64 query tokens per batch on average that are not
-   being captured, per-token adds otherwise. The results agree up to fp32
-   summation order. */
-#define SAS_BWD_WINDOW_TOKENS 2   /* per-token adds for window rows */
-#define SAS_BWD_WINDOW_KEYS 4     /* the key-major window pass */
+   rows' gradients are summed. SAS_BWD_WINDOW_TOKENS: one fp32 add per (token,
+   row, head group, channel), for every row. SAS_BWD_WINDOW_KEYS: key-major,
+   each row's gradient summed over the tokens that attend it: by the prefill
+   path where SAS_BWD_WORKSPACE is set and sas_bwd_plan reports a workspace
+   (below); else for the window rows alone, added once per 16-head group by a
+   pass beside the per-token kernel on a side stream of the library (one per
+   device, created on first use, forked from and joined back to `stream` by
+   events; one after the other on `stream` while it is being captured).
+   Neither flag: key-major for calls with at least 64 query tokens per batch
+   on average that are not being captured, per-token adds otherwise. The
+   results agree up to fp32 summation order. */
+#define SAS_BWD_WINDOW_TOKENS 2   /* per-token adds */
+#define SAS_BWD_WINDOW_KEYS 4     /* key-major */
 /* The prefill path of sas_bwd_v1: with SAS_BWD_WORKSPACE, fwd.workspace holds
    the bytes sas_bwd_plan reports, and calls that would take the key-major
    window pass sum the compressed rows' gradients key-major too, all on
-   `stream`. With SAS_BWD_DQ_DTYPE as well, where sas_bwd_plan allows it, dq is
+   `stream` (H a multiple of 32, q and dout 16-byte aligned, num_splits 0; top-k
+   tokens with more than 7 K rows below their causal threshold add their
+   compressed rows' per token). With SAS_BWD_DQ_DTYPE as well, where sas_bwd_plan
+   allows it, dq is
    [T, H, D] in the query dtype, written whole (it need not be zeroed), and the
    path is taken under capture too. */
 #define SAS_BWD_WORKSPACE 8
