@@ -2095,16 +2095,35 @@ int win_run(const SasFwdArgs* a, const Plan& pl) {
   return (a->T * pl.nhg + cus - 1) / cus > rounds * (0.75 + 0.4 * units) ? (int)run : 0;
 }
 
-// Dense compressed calls walk runs of tokens too, where batches are long enough
-// to have runs and from four (D = 512) or eight (D = 576) rounds of 64-head
-// workgroups on: there the runs were measured faster (64 heads, ratio 128: D = 576, 512 tokens 32.6 against 28.0 us, 1000 tokens 50.6 against
-// 52.0, 2000 tokens 90 against 97, 3 x 301 tokens with 128 heads and a 64-row
-// window 86.8 against 86.1; D = 512 with 128 heads, 512 tokens 42 against 53;
-// 300 batches of 3 tokens 69 against 61).
-bool dense_runs(const SasFwdArgs* a, const Plan& pl) {
-  return a->scenario == SAS_CFA && a->kv_dtype == a->q_dtype && a->H % 64 == 0 && a->win_left + kRunTokens <= kDenseWinRows &&
-         a->K <= kDenseCmpRows && pl.nsplit == 1 && a->head_waves == 0 && a->waves == 0 && a->T >= 64 * a->B &&
-         a->T * (a->H / 64) >= (a->D == 512 ? 4LL : 8LL) * sas::device_cus();
+// Dense compressed calls walk runs of tokens too (0: they don't), where sequences
+// are long enough to have runs and from four (D = 512) or eight (D = 576) rounds
+// of 64-head workgroups on: there the runs were measured faster (64 heads, ratio
+// 128: D = 576, 512 tokens 32.6 against 28.0 us, 1000 tokens 50.6 against 52.0,
+// 2000 tokens 90 against 97; D = 512 with 128 heads, 512 tokens 42 against 53;
+// 300 batches of 3 tokens 69 against 61). A sequence of the mean length is cut
+// into equal runs, so that the rounds of them (two workgroups a CU) times a run's
+// tokens and its start (two tokens' worth) are the fewest; ceil(items / places)
+// tokens a run left a second round (20 x 128 tokens, 64 heads, D = 512: 520 runs
+// on 512 places, 149 us; now 117, per token 132). At D = 576 a token costs the
+// two kernels nearly the same, and sequences below 250 tokens decide by how full
+// their runs leave the rounds: within 5 %, 300 x 64 tokens 1155 against 1203 and
+// 100 x 64 350 against 350 (64-row window 283 against 295); beyond, 32 x 100 218
+// against 210, 16 x 200 206 against 199, 13 x 130 with 128 heads 184 against 183
+// (64-row window 160 against 152), and 7 x 150 134 against 140.
+int dense_run(const SasFwdArgs* a, const Plan& pl) {
+  const long long per = a->H / 64, cus = sas::device_cus(), slots = 2 * cus;
+  if (a->scenario != SAS_CFA || a->kv_dtype != a->q_dtype || a->H % 64 || a->win_left + kRunTokens > kDenseWinRows ||
+      a->K > kDenseCmpRows || pl.nsplit != 1 || a->head_waves != 0 || a->waves != 0 || a->T < 64 * a->B ||
+      a->T * per < (a->D == 512 ? 4 : 8) * cus)
+    return 0;
+  const long long len = a->T / a->B;
+  long long best = 1, rounds = 0, cost = LLONG_MAX;
+  for (long long run = std::min<long long>(kRunTokens, len); run >= 1; --run) {
+    const long long r = (a->B * per * ((len + run - 1) / run) + slots - 1) / slots;
+    if (r * (run + 2) < cost) { cost = r * (run + 2); best = run; rounds = r; }
+  }
+  if (a->D == 576 && len < 250 && rounds * best * slots > 1.05 * a->T * per) return 0;
+  return (int)best;
 }
 
 template <int HW, int NW, int D, typename QT, int KVF, bool EXW = false>
@@ -2262,11 +2281,9 @@ extern "C" int sas_fwd_v1(const SasFwdArgs* a, void* stream) {
   hipStream_t st = (hipStream_t)stream;
 
   if (const int run = win_run(a, pl)) return launch_fwd_win(fp, (int)a->D, a->q_dtype, run, st);
-  if (dense_runs(a, pl)) {
-    // (two dense workgroups share a CU)
-    const long long cus = 2LL * sas::device_cus(), per = a->H / 64;
-    fp.nhg = (int)per;
-    return launch_fwd_win(fp, (int)a->D, a->q_dtype, (int)std::min<long long>(kRunTokens, (a->T * per + cus - 1) / cus), st);
+  if (const int run = dense_run(a, pl)) {
+    fp.nhg = (int)a->H / 64;
+    return launch_fwd_win(fp, (int)a->D, a->q_dtype, run, st);
   }
   if (fp8) rc = dispatch_hw<576, __bf16, 1>(pl.hw, pl.nw, pl.exact, fp, nblocks, st);
   else if (a->q_dtype == SAS_DT_BF16)

@@ -845,6 +845,8 @@ def test_window_runs_bsnd_padding():
     # the limits of the run's tables (128 window rows + runs, 128 compressed), a compressed row per token
     ("limits", dict(B=1, H=64, q_lens=[1030], kv_lens=[1031], ratio=8, D=512, win=128)),
     ("ratio1_win1", dict(B=17, H=64, q_lens=[128] * 17, kv_lens=[128] * 17, ratio=1, win=0)),
+    ("ratio1_win1_d512", dict(B=17, H=64, q_lens=[128] * 17, kv_lens=[128] * 17, ratio=1, win=0, D=512)),
+    ("ratio2_win1", dict(B=9, H=64, q_lens=[256] * 9, kv_lens=[256] * 9, ratio=2, win=0)),
     ("short_kv", dict(B=2, H=64, q_lens=[800, 300], kv_lens=[350, 3], ratio=4, win=40, D=512)),
     ("short_kv_d576", dict(B=2, H=64, q_lens=[1700, 400], kv_lens=[700, 3], ratio=8, win=40)),
     ("missing_blocks", dict(B=1, H=128, q_lens=[1050], kv_lens=[1050], ratio=16, bs=16)),
@@ -1032,3 +1034,40 @@ def test_signature_in_use_is_kept(monkeypatch):
     torch.cuda.synchronize()
     assert 1 not in resolved and len(resolved) == api._CACHE_MAX + 38
     assert len(api._cache) <= api._CACHE_MAX
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,spec,runs", [
+    # sequences cut into equal runs: uneven lengths around the mean, one longer
+    # than several runs, an empty one; whole sequences of 64 tokens and more
+    ("ragged", dict(B=6, H=64, q_lens=[1, 90, 700, 0, 64, 300], kv_lens=[900, 90, 710, 5, 400, 300], ratio=16, D=512), True),
+    ("whole", dict(B=20, H=64, q_lens=[64] * 20, kv_lens=[64 + i for i in range(20)], ratio=4, D=512, win=20, bs=16), True),
+    ("d576", dict(B=3, H=128, q_lens=[250, 251, 530], kv_lens=[300, 400, 530], ratio=8), True),
+    # D = 576, sequences below 250 tokens: runs that fill their rounds (512 of
+    # 16 tokens), and one workgroup per token where they do not (494 of 7)
+    ("d576_full", dict(B=32, H=128, q_lens=[128] * 32, kv_lens=[128] * 32, ratio=16, win=30), True),
+    ("d576_short", dict(B=13, H=128, q_lens=[130] * 13, kv_lens=[140] * 13, ratio=16, win=30), False),
+])
+def test_dense_run_rule(name, spec, runs):
+    """The dense runs' length and the line to one workgroup per token against
+    that kernel (head_waves given; the same bits where the rule keeps it)."""
+    from dsv4_amd.api import prepare_sparse_attn_sharedkv
+    inp = _small(K=0, scenario=2, **spec)
+    d = inp.to("cuda")
+    kw = d.api_kwargs()
+    res = []
+    for hw in (0, 4):
+        pc = prepare_sparse_attn_sharedkv(d.q, head_waves=hw, **kw)
+        pc.out.fill_(float("nan"))
+        pc.launch()
+        torch.cuda.synchronize()
+        res.append((pc.out.float().cpu(), pc.lse.cpu()))
+    (o0, l0), (o1, l1) = res
+    assert torch.isfinite(o0).all()
+    torch.testing.assert_close(l0, l1, atol=2e-5, rtol=2e-6)
+    # each P rounds against another running maximum: a rounding step of each
+    # (2 x 2^-9 in bf16), and the output's own
+    vmax = float(max(inp.ori_kv.abs().max(), inp.cmp_kv.abs().max()))
+    assert float((o0 - o1).abs().max()) <= 2 * 2.0 ** -8 * vmax
+    assert float((o0 - o1).norm() / o1.norm()) < 2.0 ** -8
+    assert torch.equal(o0, o1) == (not runs)
