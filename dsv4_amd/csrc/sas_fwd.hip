@@ -2072,27 +2072,46 @@ int make_plan(const SasFwdArgs* a, Plan* pl) {
   return SAS_OK;
 }
 
-// Window-only calls walk runs of tokens (sas_fwd_win.hip): the tokens of a run,
-// or 0 for one workgroup per (token, head group). A run belongs to one sequence:
-// a sequence of the mean length is cut into as many equal runs as leave all
-// sequences' in one round of the CUs, or stays whole (140 sequences of 3 tokens,
-// 64 heads: runs of 3 tokens 28.7 us, of ceil(T / CUs) = 2 tokens 44.0). Runs
-// are taken where their rounds cost less: a round of them loads a whole window
-// and then works through `units` (16 heads of a token) a wave, about 0.75 + 0.4
-// units of the other kernel's round. H = 64, D = 576, per token against runs:
+// Calls over runs of tokens (sas_fwd_win.hip). A run belongs to one sequence, and
+// the sequences' lengths are on the device: B sequences of any lengths come to
+// about T / run + 0.55 B runs (whole ones: B), equal ones to fewer. A run's length
+// leaves room for that: 60 sequences of 6 to 34 tokens, 64 heads, D = 576, 16-row
+// window, cut into runs of 5 (240 if equal) were 270 runs on 256 CUs, 65 us, and
+// take 48 in runs of 7.
+long long runs_of(const SasFwdArgs* a, int run) {
+  return std::max<long long>(a->B, (a->T + run - 1) / run + (a->B - 1) * 11 / 20);
+}
+// tokens of the longest run: sequences up to twice the mean length
+long long run_tokens(const SasFwdArgs* a, int run) {
+  return a->B == 1 ? run : std::min<long long>(run, (2 * a->T + a->B - 1) / a->B);
+}
+
+// Window-only calls: the tokens of a run, or 0 for one workgroup per (token, head
+// group). The cheapest length under the costs below is taken where it beats the
+// other kernel's rounds. One-round costs in us, fitted over 16 to 128 heads, both
+// widths, windows of 1 to 128 rows and 1 to 1024 sequences: per token 9.2 + 0.05 a
+// window row (64 heads a workgroup; else 0.02); a run 7 + 0.035 a row and 0.3 +
+// 0.095 H a token. D = 576, 64 heads, per token against runs: a 128-row window,
 // one sequence of 256 / 384 / 1000 tokens 16.2 / 27.4 / 55 against 17.3 / 21.6 /
-// 39 us; 300 / 1024 sequences of one token 31 / 79 against 35 / 104 us (128
-// heads 44 / 144 against 46 / 130, 48 heads 49 / 159 against 33 / 99); of one or
-// two 35 / 126 against 41 / 112; of two 49 / 163 against 47 / 128.
+// 39; 300 sequences of one token 31 against 35 (128 heads 44 / 46, 48 heads 49 /
+// 33); a 16-row one, 13 sequences of 90 to 510 tokens 150 against 123, 239 of 8 to
+// 47 256 against 300 and more.
 int win_run(const SasFwdArgs* a, const Plan& pl) {
   if (!pl.exact || a->scenario != SAS_SWA || a->kv_dtype != a->q_dtype || a->win_left >= 128 || a->head_waves != 0)
     return 0;
   const long long cus = sas::device_cus(), len = std::max<long long>(1, a->T / a->B);
-  const long long per_seq = std::max<long long>(1, cus / a->B);
-  const long long run = std::min<long long>(kRunTokens, std::max((len + per_seq - 1) / per_seq, (a->T + cus - 1) / cus));
-  const long long rounds = (a->B * ((len + run - 1) / run) + cus - 1) / cus;
-  const double units = std::max(1.0, std::min((double)run, (double)a->T / a->B) * a->H / 64);
-  return (a->T * pl.nhg + cus - 1) / cus > rounds * (0.75 + 0.4 * units) ? (int)run : 0;
+  const double start = 7 + 0.035 * a->win_left, token = 0.3 + 0.095 * a->H;
+  double cost = (a->T * pl.nhg + cus - 1) / cus * (9.2 + (pl.hw == 4 ? 0.05 : 0.02) * a->win_left);
+  int best = 0;
+  for (int run = 1; run <= kRunTokens; ++run) {
+    const long long items = runs_of(a, run);
+    const double item = start + token * run_tokens(a, run);
+    // one round; rounds of full runs; whole sequences, evened out but for the last ones
+    const double c = items <= cus ? item : run < len ? (items + cus - 1) / cus * item
+                                                     : (items * start + a->T * token) / cus + 0.6 * item;
+    if (c < cost) { cost = c; best = run; }
+  }
+  return best;
 }
 
 // Dense compressed calls walk runs of tokens too (0: they don't), where sequences
