@@ -2114,35 +2114,32 @@ int win_run(const SasFwdArgs* a, const Plan& pl) {
   return best;
 }
 
-// Dense compressed calls walk runs of tokens too (0: they don't), where sequences
-// are long enough to have runs and from four (D = 512) or eight (D = 576) rounds
-// of 64-head workgroups on: there the runs were measured faster (64 heads, ratio
-// 128: D = 576, 512 tokens 32.6 against 28.0 us, 1000 tokens 50.6 against 52.0,
-// 2000 tokens 90 against 97; D = 512 with 128 heads, 512 tokens 42 against 53;
-// 300 batches of 3 tokens 69 against 61). A sequence of the mean length is cut
-// into equal runs, so that the rounds of them (two workgroups a CU) times a run's
-// tokens and its start (two tokens' worth) are the fewest; ceil(items / places)
-// tokens a run left a second round (20 x 128 tokens, 64 heads, D = 512: 520 runs
-// on 512 places, 149 us; now 117, per token 132). At D = 576 a token costs the
-// two kernels nearly the same, and sequences below 250 tokens decide by how full
-// their runs leave the rounds: within 5 %, 300 x 64 tokens 1155 against 1203 and
-// 100 x 64 350 against 350 (64-row window 283 against 295); beyond, 32 x 100 218
-// against 210, 16 x 200 206 against 199, 13 x 130 with 128 heads 184 against 183
-// (64-row window 160 against 152), and 7 x 150 134 against 140.
+// Dense compressed calls (0: they don't walk runs), from four rounds of 64-head
+// workgroups and 64 tokens a sequence on (D = 512), or eight and 1000 (D = 576). Two
+// runs share a CU; a token of theirs takes the two 1.64 (D = 512) or 1.76 rounds of
+// the other kernel, whatever the window and the compressed rows, 1.72 with sequences
+// below 250 tokens, where that kernel's rounds are shorter (1.7 to 2.15 below 1000
+// at D = 576: no gain), and each further round of runs one token's time. Per token
+// against runs, us, 64 heads, 128-row window, ratio 64: D = 512, one sequence of
+// 1500 tokens 78 against 59, 20 of 128 101 against 94 in runs of 6, 60 of 21 to 119
+// 158 against 166; D = 576, one of 1500 78 against 68, of 4000 225 against 206, 60
+// of 21 to 119 178 against 196; 128 heads, 23 of 20 to 113 107 against 120 in runs
+// of 7, and 149 in runs of 6, which are 1.04 rounds.
 int dense_run(const SasFwdArgs* a, const Plan& pl) {
   const long long per = a->H / 64, cus = sas::device_cus(), slots = 2 * cus;
   if (a->scenario != SAS_CFA || a->kv_dtype != a->q_dtype || a->H % 64 || a->win_left + kRunTokens > kDenseWinRows ||
       a->K > kDenseCmpRows || pl.nsplit != 1 || a->head_waves != 0 || a->waves != 0 || a->T < 64 * a->B ||
-      a->T * per < (a->D == 512 ? 4 : 8) * cus)
+      a->T * per < (a->D == 512 ? 4 : 8) * cus || (a->D == 576 && a->T < 1000 * a->B))
     return 0;
-  const long long len = a->T / a->B;
-  long long best = 1, rounds = 0, cost = LLONG_MAX;
-  for (long long run = std::min<long long>(kRunTokens, len); run >= 1; --run) {
-    const long long r = (a->B * per * ((len + run - 1) / run) + slots - 1) / slots;
-    if (r * (run + 2) < cost) { cost = r * (run + 2); best = run; rounds = r; }
+  const double token = a->D == 576 ? 1.76 : a->T < 250 * a->B ? 1.72 : 1.64;
+  double cost = (double)((a->T * per + cus - 1) / cus);
+  int best = 0;
+  for (int run = 1; run <= kRunTokens; ++run) {
+    const long long rounds = (per * runs_of(a, run) + slots - 1) / slots;
+    const double c = token * (rounds * (run_tokens(a, run) + 1) - 1);
+    if (c < cost) { cost = c; best = run; }
   }
-  if (a->D == 576 && len < 250 && rounds * best * slots > 1.05 * a->T * per) return 0;
-  return (int)best;
+  return best;
 }
 
 template <int HW, int NW, int D, typename QT, int KVF, bool EXW = false>

@@ -846,6 +846,7 @@ def test_window_runs_bsnd_padding():
     ("limits", dict(B=1, H=64, q_lens=[1030], kv_lens=[1031], ratio=8, D=512, win=128)),
     ("ratio1_win1", dict(B=17, H=64, q_lens=[128] * 17, kv_lens=[128] * 17, ratio=1, win=0)),
     ("ratio1_win1_d512", dict(B=17, H=64, q_lens=[128] * 17, kv_lens=[128] * 17, ratio=1, win=0, D=512)),
+    ("ratio16_win1", dict(B=2, H=64, q_lens=[1100] * 2, kv_lens=[1100] * 2, ratio=16, win=0)),
     ("ratio2_win1", dict(B=9, H=64, q_lens=[256] * 9, kv_lens=[256] * 9, ratio=2, win=0)),
     ("short_kv", dict(B=2, H=64, q_lens=[800, 300], kv_lens=[350, 3], ratio=4, win=40, D=512)),
     ("short_kv_d576", dict(B=2, H=64, q_lens=[1700, 400], kv_lens=[700, 3], ratio=8, win=40)),
@@ -1039,15 +1040,20 @@ def test_signature_in_use_is_kept(monkeypatch):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,spec,runs", [
-    # sequences cut into equal runs: uneven lengths around the mean, one longer
-    # than several runs, an empty one; whole sequences of 64 tokens and more
-    ("ragged", dict(B=6, H=64, q_lens=[1, 90, 700, 0, 64, 300], kv_lens=[900, 90, 710, 5, 400, 300], ratio=16, D=512), True),
-    ("whole", dict(B=20, H=64, q_lens=[64] * 20, kv_lens=[64 + i for i in range(20)], ratio=4, D=512, win=20, bs=16), True),
-    ("d576", dict(B=3, H=128, q_lens=[250, 251, 530], kv_lens=[300, 400, 530], ratio=8), True),
-    # D = 576, sequences below 250 tokens: runs that fill their rounds (512 of
-    # 16 tokens), and one workgroup per token where they do not (494 of 7)
-    ("d576_full", dict(B=32, H=128, q_lens=[128] * 32, kv_lens=[128] * 32, ratio=16, win=30), True),
+    # uneven lengths around the mean, one longer than many runs, an empty one;
+    # short sequences of equal lengths
+    ("ragged_long", dict(B=6, H=64, q_lens=[1, 90, 1500, 0, 64, 700], kv_lens=[900, 90, 1510, 5, 400, 700], ratio=16, D=512), True),
+    ("cut_64", dict(B=75, H=64, q_lens=[64] * 75, kv_lens=[64 + i for i in range(75)], ratio=4, D=512, win=20, bs=16), True),
+    ("d576_long", dict(B=3, H=64, q_lens=[1, 1400, 1650], kv_lens=[300, 1500, 1650], ratio=16), True),
+    # one workgroup per token: five rounds of them are the runs' time
+    ("ragged", dict(B=6, H=64, q_lens=[1, 90, 700, 0, 64, 300], kv_lens=[900, 90, 710, 5, 400, 300], ratio=16, D=512), False),
+    ("whole", dict(B=20, H=64, q_lens=[64] * 20, kv_lens=[64 + i for i in range(20)], ratio=4, D=512, win=20, bs=16), False),
+    # sequences below 1000 tokens at D = 576, equal and ragged ones
+    ("d576", dict(B=3, H=128, q_lens=[250, 251, 530], kv_lens=[300, 400, 530], ratio=8), False),
+    ("d576_full", dict(B=32, H=128, q_lens=[128] * 32, kv_lens=[128] * 32, ratio=16, win=30), False),
     ("d576_short", dict(B=13, H=128, q_lens=[130] * 13, kv_lens=[140] * 13, ratio=16, win=30), False),
+    ("d576_ragged", dict(B=23, H=128, q_lens=[(20, 67, 113, 46, 87)[i % 5] for i in range(23)],
+                         kv_lens=[120] * 23, ratio=8), False),
 ])
 def test_dense_run_rule(name, spec, runs):
     """The dense runs' length and the line to one workgroup per token against
