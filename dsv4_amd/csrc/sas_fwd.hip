@@ -2100,6 +2100,7 @@ int win_run(const SasFwdArgs* a, const Plan& pl) {
   if (!pl.exact || a->scenario != SAS_SWA || a->kv_dtype != a->q_dtype || a->win_left >= 128 || a->head_waves != 0)
     return 0;
   const long long cus = sas::device_cus(), len = std::max<long long>(1, a->T / a->B);
+  if (a->T * pl.nhg <= cus) return 0;   // one round: a run loads as many rows as a token
   const double start = 7 + 0.035 * a->win_left, token = 0.3 + 0.095 * a->H;
   double cost = (a->T * pl.nhg + cus - 1) / cus * (9.2 + (pl.hw == 4 ? 0.05 : 0.02) * a->win_left);
   int best = 0;

@@ -981,6 +981,7 @@ def test_runs_without_a_sink_and_with_missing_rows(name, spec):
     ("one_token_h64", dict(B=300, H=64, q_lens=[1] * 300, kv_lens=[60 + i for i in range(300)]), False),
     ("one_token_h16_d512", dict(B=300, H=16, q_lens=[1] * 300, kv_lens=[140] * 300, D=512), False),
     ("ragged_small_window", dict(B=230, H=64, q_lens=[(2, 5, 10, 4, 8)[i % 5] for i in range(230)], kv_lens=[40] * 230, win=15), False),
+    ("one_round_h16", dict(B=200, H=16, q_lens=[1] * 200, kv_lens=[60] * 200, win=3), False),
     ("one_round", dict(B=2, H=64, q_lens=[200, 56], kv_lens=[200, 300]), False),
     # runs: one-token sequences of many head groups, whole short sequences,
     # sequences around and beyond the mean length, a padded empty one
